@@ -380,6 +380,10 @@ int vkhip_gemm_noalloc(const float* a, const vkhip_operand* a_desc,
  * no split) and chunk (K-tiles per partition, a power of two). */
 int vkhip_gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k,
                     int32_t split_request, uint32_t* out_splits, uint32_t* out_chunk);
+/* 1 when AUTO gives the M x N product A @ B and the N x M product B^T @ A^T
+ * over the same K the same bits (equal plans, and a kernel whose sums do not
+ * depend on which operand comes first), else 0. Callable without a GPU. */
+int vkhip_gemm_transposable(uint32_t batch, uint32_t m, uint32_t n, uint32_t k);
 
 /* dst[i] = carry-stack fold of ws[s*ne + i], s = 0..splits-1
  * (reference gemm_split_k_reduce.comp:48-85). Deterministic, bit-stable. */

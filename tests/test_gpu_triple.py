@@ -1,0 +1,118 @@
+"""Products on the bf16 matrix cores (gemm_triple.h): three-term operands, all
+layouts the same bits, and the fp32 pass for what the terms cannot hold."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import SEED, gemm_tolerance, normwise_rel_err
+from vkml_amd import ops
+from vkml_amd.device import DeviceArray
+
+pytestmark = pytest.mark.gpu
+
+
+def _view(x: np.ndarray, how: str) -> DeviceArray:
+    """x as a device view: "n" as it lies, "t" stored transposed, "o" inside a
+    wider array at an odd offset (rows at any float address), "r" its columns
+    stored last to first."""
+    swap = list(range(x.ndim - 2)) + [x.ndim - 1, x.ndim - 2]
+    if how == "t":
+        return DeviceArray.from_numpy(np.ascontiguousarray(x.transpose(swap))).transpose(-2, -1)
+    if how == "r":
+        d = DeviceArray.from_numpy(np.ascontiguousarray(x[..., ::-1]))
+        return DeviceArray(d.shape, d.dtype, d.strides[:-1] + (-1,), d.buffer, x.shape[-1] - 1)
+    if how == "o":
+        wide = np.full(x.shape[:-1] + (x.shape[-1] + 3,), np.nan, np.float32)
+        wide[..., 1:-2] = x
+        d = DeviceArray.from_numpy(wide)
+        return DeviceArray(x.shape, d.dtype, d.strides, d.buffer, 1)
+    return DeviceArray.from_numpy(x)
+
+
+# (batch, m, n, k): 64, 128 and 256 tiles; one row or column past a tile, less
+# than four rows in the last tile, a last stage of 1, 9 and 15 k, split K
+SHAPES = [(1, 1000, 1501, 777), (1, 257, 2049, 1025), (1, 4099, 3841, 89), (3, 515, 641, 319),
+          (1, 67, 130, 40001), (1, 33, 4100, 2100), (16, 129, 131, 1040)]
+
+
+@pytest.mark.parametrize("batch,m,n,k", SHAPES)
+def test_layouts_and_edges(hip, batch, m, n, k):
+    rng = np.random.default_rng(SEED + m + n + k)
+    lead = (batch,) if batch > 1 else ()
+    a = rng.standard_normal(lead + (m, k), dtype=np.float32)
+    b = rng.standard_normal(lead + (k, n), dtype=np.float32)
+    print(f"triple {batch} {m}x{n}x{k}", flush=True)
+    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    rows = np.unique(np.r_[0:4, m // 2, m - 4:m])
+    exact = a[..., rows, :].astype(np.float64) @ b.astype(np.float64)
+    assert normwise_rel_err(got[..., rows, :], exact) <= min(gemm_tolerance(k), 2.0 ** -23 * np.sqrt(k))
+    for la, lb in (("n", "t"), ("t", "n"), ("t", "t"), ("o", "o"), ("r", "n"), ("n", "r")):
+        same = ops.matmul(_view(a, la), _view(b, lb)).numpy()
+        differ = int(np.count_nonzero(same.view(np.uint32) != got.view(np.uint32)))
+        assert differ == 0, (la, lb)
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 700, 600), (2100, 2300, 100)])
+@pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1e36), (1e30, 1e-30), (3e-39, 1.0), (1e-20, 1e-19)])
+def test_scales_keep_fp32_accuracy(hip, m, n, k, scale_a, scale_b):
+    """Operands of any fp32 scale, subnormals included: the fp32 product's
+    accuracy (relative, or one part in 2^24 of the smallest normal number)."""
+    rng = np.random.default_rng(SEED + m)
+    a = (rng.standard_normal((m, k)) * scale_a).astype(np.float32)
+    b = (rng.standard_normal((k, n)) * scale_b).astype(np.float32)
+    print(f"triple scale {scale_a} {scale_b}", flush=True)
+    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy().astype(np.float64)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    off = np.linalg.norm(got - exact)
+    assert off <= 2.0 ** -23 * np.sqrt(k) * np.linalg.norm(exact) + 2.0 ** -149 * k * np.sqrt(m * n)
+
+
+def test_infinities_nans_and_the_largest_values(hip):
+    """Where a 64-bit product is finite in fp32, the result is it; elsewhere
+    infinities and NaNs land where IEEE arithmetic puts them."""
+    rng = np.random.default_rng(SEED)
+    m, n, k = 600, 640, 800
+    a = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
+    b = rng.uniform(0.5, 1.5, (k, n)).astype(np.float32)
+    a[3, 5] = np.inf
+    a[70, 9] = -np.inf
+    b[11, 200] = np.nan
+    a[130, :] = 0.0
+    a[130, 7] = np.finfo(np.float32).max  # rounds up to infinity as a bf16
+    b[7, 300] = 0.5
+    b[20, 64] = np.inf
+    a[200, 20] = 0.0                      # 0 * inf
+    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        exact = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exact))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(exact))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(exact))
+    fine = np.isfinite(exact)
+    np.testing.assert_allclose(got[fine], exact[fine], rtol=1e-5)
+
+
+@pytest.mark.parametrize("n,c,hw,cout,window,stride", [(37, 40, (19, 23), 70, 3, 1), (9, 65, (30, 31), 130, 5, 2),
+                                                      (64, 33, (32, 32), 257, 3, 1)])
+def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stride):
+    rng = np.random.default_rng(SEED + c)
+    x = rng.uniform(-1, 1, (n, c) + hw).astype(np.float32)
+    w = rng.uniform(-0.1, 0.1, (cout, c, window, window)).astype(np.float32)
+    dx, dw = DeviceArray.from_numpy(x), DeviceArray.from_numpy(w)
+    pad = window // 2
+    print(f"triple conv {x.shape} {cout}", flush=True)
+    cols = ops.im2col(dx, window, stride, pad)
+    _, ck, L = cols.shape
+    got = ops.conv2d(dx, dw, stride, pad)
+    want = ops.matmul(dw.reshape(1, 1, cout, ck).broadcast_to((1, n, cout, ck)), cols.reshape(1, n, ck, L))
+    assert np.array_equal(got.numpy().reshape(-1), want.numpy().reshape(-1))
+    g = rng.standard_normal(got.shape).astype(np.float32)
+    dg = DeviceArray.from_numpy(g)
+    per = ops.conv2d_weight_grad(dx, dg, window, stride, pad)
+    want = ops.matmul(dg.reshape(1, n, cout, L), cols.reshape(1, n, ck, L).transpose(-2, -1)).numpy()
+    assert np.array_equal(per.numpy().reshape(-1), want.reshape(-1))
+    total = ops.conv2d_weight_grad_sum(dx, dg, window, stride, pad).numpy()
+    exact = np.einsum("nol,nkl->ok", g.reshape(n, cout, L).astype(np.float64), cols.numpy().astype(np.float64),
+                      optimize=True)
+    assert normwise_rel_err(total, exact) <= 2.0 ** -23 * np.sqrt(n * L)

@@ -150,6 +150,7 @@ SIGNATURES = {
                                            POINTER(c_size_t)]),
     "vkhip_gemm_plan": (c_int, [c_uint32, c_uint32, c_uint32, c_uint32, c_int32,
                                 POINTER(c_uint32), POINTER(c_uint32)]),
+    "vkhip_gemm_transposable": (c_int, [c_uint32, c_uint32, c_uint32, c_uint32]),
     "vkhip_split_k_reduce": (c_int, [c_void_p, c_void_p, c_uint64, c_uint32]),
     "vkhip_gemv": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_uint32, c_uint32]),
     "vkhip_im2col": (c_int, [c_void_p, POINTER(Operand), c_void_p, POINTER(Unfold)]),

@@ -26,8 +26,10 @@ LIBDIR = PKG / "lib"
 LIB = LIBDIR / "libvkhip.so"
 OBJDIR = ROOT / "_build" / "vkhip"
 
-SOURCES = ["runtime.hip", "allocator.hip", "observe.hip", "program.hip", "gemm.hip", "movement.hip",
-           "reduce.hip", "elementwise.hip", "conv_small.hip"]
+SOURCES = ["runtime.hip", "allocator.hip", "observe.hip", "program.hip", "gemm.hip",
+           "gemm_triple_256x128.hip",
+           "gemm_triple_128x128.hip", "gemm_triple_64x64.hip",
+           "movement.hip", "reduce.hip", "elementwise.hip", "conv_small.hip"]
 
 
 def hipcc() -> str:

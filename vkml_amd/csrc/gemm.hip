@@ -19,102 +19,14 @@
 //   - inside a K-tile, lane half h (lanes 32..63) supplies k in the upper half
 //     of the tile, so each lane's k values are contiguous in LDS. The sum over
 //     k is unchanged; only the order MFMA visits the k values differs.
-#include "common.h"
+#include "gemm_triple.h"
 #include "conv_small.h"
 
+#include <cmath>
 #include <mutex>
 #include <vector>
 
 namespace vkhip {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// An epilogue adds bias[(i % ncols) * bias_stride] to the folded value and
-// then applies relu (v <= 0 ? 0 : v) when asked -- the ADD and RELU nodes'
-// arithmetic on the product's output -- or (mask != null) takes the relu
-// gradient mask[i] <= 0 ? +0 : v, mask laid out as the output (RELU_BACKWARD
-// with the product as its incoming gradient; a NaN mask passes v).
-struct FoldEpilogue {
-    const float* bias;
-    int64_t bias_stride;
-    uint32_t ncols, relu;
-    const float* mask;
-};
-
-__device__ __forceinline__ float apply_epilogue(const FoldEpilogue& epi, uint64_t i, float v) {
-    if (epi.bias) {
-        v = v + epi.bias[static_cast<int64_t>(i % epi.ncols) * epi.bias_stride];
-        if (epi.relu) v = v <= 0.0f ? 0.0f : v;
-    }
-    if (epi.mask && epi.mask[i] <= 0.0f) v = 0.0f;
-    return v;
-}
-
-struct GemmArgs {
-    const float* a;
-    const float* b;
-    float* c;
-    int64_t sa0, sa1, sam, sak;  // A strides: batch0, batch1, m, k (elements)
-    int64_t sb0, sb1, sbk, sbn;  // B strides: batch0, batch1, k, n
-    uint32_t b1;                 // extent of batch axis 1
-    uint32_t m, n, k;
-    uint32_t tiles_m, tiles_n;
-    uint32_t ktiles;             // ceil(K / BK)
-    uint32_t chunk;              // K-tiles per split partition
-    uint64_t split_stride;       // elements between partition slices of c
-    uint32_t a_vec, b_vec;       // 16-byte loads along k are legal
-    uint32_t flat_splits;        // > 0: split grid launched flat, grid.x = tiles * flat_splits
-    uint32_t pairs;              // paired direct kernel: partition pairs per tile
-    // Convolution epilogue (unsplit register-path conv kernel only): out =
-    // acc + bias[row * bias_stride] when bias is set, then relu (x <= 0 ? 0 :
-    // x) when relu is set -- the ADD and RELU nodes' arithmetic.
-    const float* bias;
-    int64_t bias_stride;
-    uint32_t relu;
-    // A product's epilogue (MATMUL_BIAS, MATMUL_RELU_BACKWARD) applied by the
-    // kernel that writes the output (unsplit plans; split plans: the fold).
-    FoldEpilogue epi;
-};
-
-// The product epilogue at output (z, row, col), when the launch has one.
-__device__ __forceinline__ float product_epilogue(const GemmArgs& g, uint32_t z, uint32_t row,
-                                                  uint32_t col, float v) {
-    if (!g.epi.bias && !g.epi.mask) return v;
-    return apply_epilogue(g.epi, (static_cast<uint64_t>(z) * g.m + row) * g.n + col, v);
-}
-
-// Output tile (tm, tn) and K partition of this workgroup.
-//  - Unsplit grids (blockIdx.x = tile): the hardware deals workgroups to the
-//    8 XCDs round-robin, so the tile index is remapped to give each XCD a
-//    contiguous tile range, walked in groups of 8 tile-rows for L2 reuse.
-//  - Split grids launched flat (flat_splits > 0, grid.x = tiles * partitions):
-//    the workgroups one XCD receives (linear id % 8) take a contiguous range
-//    of (partition, tile) pairs, so the tiles of one partition, which read the
-//    same K slices of A and B, share that XCD's L2 instead of each fetching
-//    them from memory.
-//  - Otherwise blockIdx.y is the partition.
-// Which workgroup computes what never changes what it computes: same bits.
-__device__ __forceinline__ void tile_of(const GemmArgs& g, uint32_t& tm, uint32_t& tn,
-                                        uint32_t& split) {
-    const uint32_t ntiles = g.tiles_m * g.tiles_n;
-    uint32_t bid = blockIdx.x;
-    split = blockIdx.y;
-    if (g.flat_splits) {
-        const uint32_t total = ntiles * g.flat_splits;
-        const uint32_t xcd = bid & 7u, slot = bid >> 3, q = total >> 3, r = total & 7u;
-        const uint32_t v = xcd * q + min(xcd, r) + slot;
-        split = v / ntiles;
-        bid = v - split * ntiles;
-    } else if ((ntiles & 7u) == 0) {
-        bid = (bid & 7u) * (ntiles >> 3) + (bid >> 3);
-    }
-    const uint32_t group_span = 8u * g.tiles_n;
-    const uint32_t first_m = (bid / group_span) * 8u;
-    const uint32_t gsize = min(g.tiles_m - first_m, 8u);
-    tm = first_m + (bid % group_span) % gsize;
-    tn = (bid % group_span) / gsize;
-}
 
 // Loads one BK-deep tile of an operand (rows x BK) into registers as groups of
 // four consecutive k, then stores each group to LDS [row][k] as 16 bytes.
@@ -160,84 +72,6 @@ __host__ __device__ __forceinline__ uint32_t kcd_slot_offset(int slot, int64_t s
     return gr < rows && gk < kdim ? static_cast<uint32_t>((static_cast<int64_t>(gr) * s_row + gk) * 4)
                                   : 0x80000000u;
 }
-
-// The B operand of a convolution read straight from the image (implicit
-// im2col): element (row, pos) of image n's cols matrix [C*kh*kw, out_h*out_w]
-// is x[n, c, h, w] with row = c*kh*kw + ki*kw + kj, pos = oh*out_w + ow,
-// h = oh*stride_h - pad_h + ki*dil_h, w = ow*stride_w - pad_w + kj*dil_w, and
-// 0 outside the image (kernels_movement.cpp:438-483, the im2col kernel's map).
-struct Im2colB {
-    const float* x;  // image 0
-    int64_t sn;      // image (batch) stride in elements
-    // Within one image every offset fits 32 bits (checked by make_im2col).
-    int32_t sc, sh, sw;  // channel, row and column strides in elements
-    int32_t H, W, kh, kw, kk, strh, strw, padh, padw, dilh, dilw, ow;
-    FastDiv div_kk, div_kw, div_ow;  // by kh*kw, kw, out_w
-    const int32_t* rows;             // row table (see below)
-    uint32_t L, images;              // IMGTB: positions per image, images
-    FastDiv div_L;                   // IMGTB: by L
-};
-
-// The map splits into a part that depends only on the output position (one
-// per lane, fixed for the whole kernel) and a part that depends only on the
-// cols row (the same for every lane of a wave in the loader below). Whether
-// an element is inside the image depends on the position and on the row's
-// window element r = ki*kw + kj only: each position keeps a bit mask over r
-// of the elements that fall in the padding.
-constexpr int kMaxWindow = 63;  // kh*kw; bit 63 marks rows past K
-
-struct ImgPos {
-    int32_t h0, w0;    // top-left image coordinate of the window
-    int32_t base;      // its offset (may lie outside the image)
-    uint64_t outside;  // bit r set: window element r lies in the padding
-};
-
-__host__ __device__ __forceinline__ ImgPos img_pos(const Im2colB& g, uint32_t pos, bool valid) {
-    const uint32_t oh = g.div_ow.div(pos);
-    const uint32_t ow = pos - oh * static_cast<uint32_t>(g.ow);
-    ImgPos p;
-    p.h0 = static_cast<int32_t>(oh) * g.strh - g.padh;
-    p.w0 = static_cast<int32_t>(ow) * g.strw - g.padw;
-    p.base = p.h0 * g.sh + p.w0 * g.sw;
-    p.outside = ~0ull;
-    if (valid) {
-        for (int ki = 0; ki < g.kh; ++ki) {
-            const bool row_in = static_cast<uint32_t>(p.h0 + ki * g.dilh) < static_cast<uint32_t>(g.H);
-            for (int kj = 0; kj < g.kw; ++kj) {
-                const bool in = row_in && static_cast<uint32_t>(p.w0 + kj * g.dilw) <
-                                              static_cast<uint32_t>(g.W);
-                if (in) p.outside &= ~(1ull << (ki * g.kw + kj));
-            }
-        }
-    }
-    return p;
-}
-
-// The row part of cols row `row` (channel c, window element ki, kj): its
-// offset and its window element.
-struct ImgRow {
-    int32_t off, r;
-};
-
-__host__ __device__ __forceinline__ ImgRow img_row(const Im2colB& g, uint32_t row) {
-    const uint32_t c = g.div_kk.div(row);
-    const uint32_t r = row - c * static_cast<uint32_t>(g.kk);
-    const uint32_t ki = g.div_kw.div(r);
-    const uint32_t kj = r - ki * static_cast<uint32_t>(g.kw);
-    ImgRow q;
-    q.off = static_cast<int32_t>(c) * g.sc + static_cast<int32_t>(ki) * g.dilh * g.sh +
-            static_cast<int32_t>(kj) * g.dilw * g.sw;
-    q.r = static_cast<int32_t>(r);
-    return q;
-}
-
-// The gather reads the row part from a table built once per geometry:
-// groups of 16 rows as {4*off[16], r[16]} (byte offsets), padded past K with
-// rows whose r = 63 is outside for every position, so the loader needs no K
-// bound. The table is read through the constant address space: a wave's rows
-// are uniform, so these are scalar loads.
-constexpr int kRowGroup = 16;
-typedef const int32_t __attribute__((address_space(4)))* RowTable;
 
 template <int R, int BK, int MODE>
 struct TileLoader {
@@ -2468,6 +2302,100 @@ int gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k, int32_t split_
     return VKHIP_OK;
 }
 
+// ---- products on the bf16 matrix cores (gemm_triple.h) --------------------------
+// Whether an AUTO product runs there, on which square tile, and how many
+// consecutive partitions of its split-K plan each workgroup takes as one chain
+// (`run`; run * chunk K-tiles, slices = ceil(splits / run) partials).
+struct TriplePlan {
+    int tile = -1;  // kTripleTiles; negative: the fp32 matrix cores
+    uint32_t slices = 1, chunk = 1;
+    explicit operator bool() const { return tile >= 0; }
+};
+
+// The tiles, and microseconds per 16-deep stage of one workgroup, measured: a
+// launch of few workgroups takes `one`, a workgroup on every CU `full`, several
+// on each `share` apiece. (Per unit of work the 256x128 tile is the fastest and
+// the 64x64 tile the slowest, 4096^3 645, 690 and 915 us, so size is traded for
+// CUs left idle: 2048^3 125, 96 and 125 us, 1024^3 64, 43 and 20 us.)
+struct TripleTileTimes {
+    uint32_t bm, bn;
+    double one, full, share;
+    const char* name;
+};
+static const TripleTileTimes kTripleTiles[] = {{64, 64, 0.20, 0.285, 0.225, "64x64 tiles"},
+                                               {128, 128, 0.55, 0.75, 0.69, "128x128 tiles"},
+                                               {256, 128, 0.90, 1.27, 1.27, "256x128 tiles"}};
+
+// Microseconds of a launch of `tiles` x `slices` workgroups of `stages` stages.
+static double triple_time(const TripleTileTimes& t, uint64_t tiles, uint32_t slices, uint32_t stages,
+                          uint64_t out_elems, double cus) {
+    const double w = static_cast<double>(tiles) * slices / cus;
+    const double per = w <= 1.0 ? t.one + (t.full - t.one) * w : t.share * std::ceil(w);
+    const double fold = slices > 1 ? 4.5 + 8.0 * slices * static_cast<double>(out_elems) / 5e6 : 0.0;
+    return 4.0 + stages * per + fold;
+}
+
+constexpr double kTripleMinMacs = 268435456.0;
+
+static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
+    TriplePlan best;
+    if (m <= 32 || n <= 32 || k < 64) return best;
+    const double macs = static_cast<double>(batch) * m * n * k;
+    if (macs < kTripleMinMacs) return best;
+    uint32_t splits, chunk;
+    TileChoice plan;
+    gemm_plan(batch, m, n, k, 0, splits, chunk, plan, true);
+    // no more partials than the fp32 kernels of the same plan write: pairs of
+    // partitions there leave one, and two partitions of 64x64 tiles none
+    const uint32_t most = plan.pair ? (splits + 1) / 2 : splits == 2 && plan.bm == 64 ? 1u : splits;
+    const double cus = ctx().ready ? ctx().caps.compute_units : 256.0;
+    const uint64_t out_elems = static_cast<uint64_t>(batch) * m * n;
+    const uint32_t ktotal = ceil_div(k, 16u);
+    double best_us = 1e30;
+    for (int tile = 0; tile < 3; ++tile) {
+        const TripleTileTimes& tt = kTripleTiles[tile];
+        const uint64_t tiles = static_cast<uint64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch;
+        // slice counts about 1.4 apart: 1, 2, 3, 4, 6, 8, 12, ...
+        for (uint32_t want = 1; want <= most; want = want == 1 ? 2 : (want & (want - 1)) == 0 ? want * 3 / 2 : want / 3 * 4) {
+            const uint32_t run = (splits + want - 1) / want;
+            const uint32_t slices = (splits + run - 1) / run;
+            const uint32_t stages = std::min(ktotal, 2 * run * chunk);
+            const double us = triple_time(tt, tiles, slices, stages, out_elems, cus);
+            if (us < best_us) {
+                best_us = us;
+                best.tile = tile;
+                best.slices = slices;
+                best.chunk = run * chunk;
+            }
+        }
+    }
+    return best;
+}
+
+// Launches a product planned there; g holds the operands, strides and sizes,
+// and when the plan has one slice the epilogue. `c` is the output of one slice
+// or the partials of several.
+static int launch_triple_product(GemmArgs& g, const Im2colB& im, const TriplePlan& t, uint32_t batch, int am, int bm) {
+    g.tiles_m = ceil_div(g.m, kTripleTiles[t.tile].bm);
+    g.tiles_n = ceil_div(g.n, kTripleTiles[t.tile].bn);
+    g.chunk = t.chunk;
+    const uint64_t flat = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * t.slices;
+    if (flat > 0x7fffffffull) return fail(VKHIP_ERR_UNSUPPORTED, "gemm: %llu workgroups", static_cast<unsigned long long>(flat));
+    g.flat_splits = t.slices > 1 ? t.slices : 0;
+    const dim3 grid(static_cast<uint32_t>(flat), 1, batch);
+    return t.tile == 0   ? launch_triple_64x64(g, im, grid, am, bm)
+           : t.tile == 1 ? launch_triple_128x128(g, im, grid, am, bm)
+                         : launch_triple_256x128(g, im, grid, am, bm);
+}
+
+// How a plain operand of rows x k (strides s_row, s_k) is staged: unit k or row
+// stride with 32-bit byte offsets, else by 4-byte loads.
+static int triple_mode(uint32_t rows, uint32_t k, int64_t s_row, int64_t s_k) {
+    if (s_k == 1 && s_row >= 0 && ((static_cast<int64_t>(rows) - 1) * s_row + k) * 4 < (int64_t{1} << 31)) return TK;
+    if (s_row == 1 && s_k >= 0 && (16 * s_k + rows) * 4 < (int64_t{1} << 31)) return TR;
+    return TG;
+}
+
 template <int BMODE, int LV>
 static void launch_exact4_lv(const GemmArgs& g, uint32_t batch, int depth, const ExactImg& im,
                              int a_kfast, int b_kfast, int slog) {
@@ -2676,6 +2604,16 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
     uint32_t splits, chunk;
     TileChoice tile;
     gemm_plan(static_cast<uint32_t>(batch), m, n, k, split_req, splits, chunk, tile, true);
+    auto partials = [&](size_t need, float** ws) -> int {
+        if (!scratch) return workspace(need, ws);
+        if (need > scratch->bytes)
+            return fail(VKHIP_ERR_INVALID,
+                        "matmul %ux%ux%u (batch %llu) splits K into %u partitions whose partials "
+                        "need %zu bytes; the allocation-free entry point's scratch holds %zu",
+                        m, n, k, static_cast<unsigned long long>(batch), splits, need, scratch->bytes);
+        *ws = scratch->ptr;
+        return VKHIP_OK;
+    };
     {
         const int64_t cus = ctx().ready ? ctx().caps.compute_units : 256;
         publish("matmul.kernel", "matmul", tile.bm == 128 ? "gemm_mfma_128x128" : "gemm_mfma_64x64",
@@ -2724,6 +2662,27 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
                   : (g.sbn == 1 && aligned(b, g.sb0, g.sb1, g.sbk));
 
     const uint64_t out_elems = batch * m * n;
+    if (split_req == 0) {
+        const TriplePlan t = triple_plan(static_cast<uint32_t>(batch), m, n, k);
+        if (t) {
+            publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, t.chunk, t.slices);
+            float* target = c;
+            if (t.slices > 1) {
+                const int st = partials(out_elems * t.slices * sizeof(float), &target);
+                if (st != VKHIP_OK) return st;
+                g.split_stride = out_elems;
+            } else {
+                g.epi = fe;
+            }
+            *fused = true;
+            g.c = target;
+            int am = triple_mode(m, k, g.sam, g.sak), bm = triple_mode(n, k, g.sbn, g.sbk);
+            if (am == TG || bm == TG) am = bm = TG;
+            const int st = launch_triple_product(g, Im2colB{}, t, static_cast<uint32_t>(batch), am, bm);
+            if (st != VKHIP_OK || t.slices == 1) return st;
+            return launch_split_k_reduce(target, c, out_elems, t.slices, fe);
+        }
+    }
     int amode = akc ? (g.a_vec ? KCV : KCS) : (g.a_vec ? RCV : RCS);
     // The buffer-load paths (straight-to-LDS operands and the direct kernels)
     // address an operand by unsigned 32-bit byte offsets from its base, so
@@ -2804,19 +2763,8 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
     float* target = c;
     if (slices > 1) {
         float* ws = nullptr;
-        const size_t need = out_elems * slices * sizeof(float);
-        if (scratch) {
-            if (need > scratch->bytes)
-                return fail(VKHIP_ERR_INVALID,
-                            "matmul %ux%ux%u (batch %llu) splits K into %u partitions whose partials "
-                            "need %zu bytes; the allocation-free entry point's scratch holds %zu",
-                            m, n, k, static_cast<unsigned long long>(batch), splits, need,
-                            scratch->bytes);
-            ws = scratch->ptr;
-        } else {
-            const int wst = workspace(need, &ws);
-            if (wst != VKHIP_OK) return wst;
-        }
+        const int wst = partials(out_elems * slices * sizeof(float), &ws);
+        if (wst != VKHIP_OK) return wst;
         target = ws;
         g.split_stride = out_elems;
     }
@@ -3682,6 +3630,10 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
 
     const uint64_t out_elems = batch * m * n;
     float* target = out;
+    // the plan gemm() takes for the same product, so the same bits
+    const TriplePlan triple = triple_mode(m, k, g.sam, g.sak) == TK
+                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
+    if (triple) splits = triple.slices;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -3711,7 +3663,11 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     const uint64_t cus = ctx().ready ? static_cast<uint64_t>(ctx().caps.compute_units) : 256u;
     const uint64_t w128 = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * splits * batch;
     const uint64_t w64 = static_cast<uint64_t>(g.tiles_m) * ceil_div(n, 64) * splits * batch;
-    if (tile.bm == 128 && 0.94 * round_fill(w64, 2 * cus) > round_fill(w128, 2 * cus)) {
+    if (triple) {
+        publish("matmul.operands", "conv2d", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
+                triple.chunk, triple.slices);
+        st = launch_triple_product(g, im, triple, static_cast<uint32_t>(batch), TK, TI);
+    } else if (tile.bm == 128 && 0.94 * round_fill(w64, 2 * cus) > round_fill(w128, 2 * cus)) {
         g.tiles_n = ceil_div(n, 64);
         st = launch_conv_tiles<128, 64, 64, 32, IMG>(g, im, static_cast<uint32_t>(batch), splits, amode);
     } else if (tile.bm == 128)
@@ -3845,6 +3801,9 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     const int amode = a_kcd ? KCD : (g.a_vec ? KCV : KCS);
     const uint64_t out_elems = batch * m * n;
     float* target = out;
+    const TriplePlan triple = g.sa1 >= 0 && triple_mode(m, k, g.sam, g.sak) == TK && triple_image_fits(im, oh)
+                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
+    if (triple) splits = triple.slices;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -3854,7 +3813,11 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     g.c = target;
     g.split_stride = splits > 1 ? out_elems : 0;
     int st;
-    if (tile.bm == 128 && wgrad_direct_fits(g, k, target)) {
+    if (triple) {
+        publish("matmul.operands", "conv2d_weight_grad", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
+                triple.chunk, triple.slices);
+        st = launch_triple_product(g, im, triple, static_cast<uint32_t>(batch), TK, TT);
+    } else if (tile.bm == 128 && wgrad_direct_fits(g, k, target)) {
         // both operands straight into LDS (same bits as the register path);
         // 128x64 tiles when their rounds fill the machine better (as in gemm())
         const bool narrow = wgrad_narrow_tiles(g, splits, batch);
@@ -4112,6 +4075,10 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     const int amode = g.a_vec ? KCV : KCS;
     const uint64_t out_elems = static_cast<uint64_t>(m) * n;
     float* target = out;
+    const TriplePlan triple = g.sa1 >= 0 && triple_mode(m, static_cast<uint32_t>(L), g.sam, g.sak) == TK &&
+                                      triple_image_fits(im, oh)
+                                  ? triple_plan(1, m, n, k) : TriplePlan{};
+    if (triple) splits = triple.slices;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -4121,7 +4088,11 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     g.c = target;
     g.split_stride = splits > 1 ? out_elems : 0;
     int st;
-    if (tile.bm == 128 && wgrad_direct_fits(g, static_cast<uint32_t>(L), target)) {
+    if (triple) {
+        publish("matmul.operands", "conv2d_weight_grad_sum", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
+                triple.chunk, triple.slices);
+        st = launch_triple_product(g, im, triple, 1, TKB, TTB);
+    } else if (tile.bm == 128 && wgrad_direct_fits(g, static_cast<uint32_t>(L), target)) {
         const bool narrow = wgrad_narrow_tiles(g, splits, 1);
         if (narrow) g.tiles_n = ceil_div(n, 64u);
         const uint64_t flat = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * splits;
@@ -4307,6 +4278,15 @@ extern "C" int vkhip_gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t 
     if (out_splits) *out_splits = s;
     if (out_chunk) *out_chunk = c;
     return VKHIP_OK;
+}
+
+extern "C" int vkhip_gemm_transposable(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
+    uint32_t s, c, s2, c2;
+    vkhip::TileChoice t;
+    vkhip::gemm_plan(batch, m, n, k, 0, s, c, t, true);
+    vkhip::gemm_plan(batch, n, m, k, 0, s2, c2, t, true);
+    // (the triple kernels add A's lower terms and B's in a fixed order)
+    return s == s2 && c == c2 && !vkhip::triple_plan(batch, m, n, k) && !vkhip::triple_plan(batch, n, m, k);
 }
 
 extern "C" int vkhip_split_k_reduce(const float* ws, float* dst, uint64_t ne, uint32_t splits) {
