@@ -2335,13 +2335,17 @@ static double triple_time(const TripleTileTimes& t, uint64_t tiles, uint32_t sli
     return 4.0 + stages * per + fold;
 }
 
+// Products of more than this many multiply-adds take them. Below, the launch
+// and the first loads are most of the time on either path: 128x8192x256 (2^28)
+// 10.7 us on the fp32 cores and 11.0 here, 1000x1000x64 11.1 and 11.0, 512^3
+// 11.4 and 12.6; above, 700^3 17.1 and 16.4, 1024^3 24.7 and 20.7.
 constexpr double kTripleMinMacs = 268435456.0;
 
 static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
     TriplePlan best;
     if (m <= 32 || n <= 32 || k < 64) return best;
     const double macs = static_cast<double>(batch) * m * n * k;
-    if (macs < kTripleMinMacs) return best;
+    if (macs <= kTripleMinMacs) return best;
     uint32_t splits, chunk;
     TileChoice plan;
     gemm_plan(batch, m, n, k, 0, splits, chunk, plan, true);

