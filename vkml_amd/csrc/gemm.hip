@@ -1323,150 +1323,111 @@ __global__ __launch_bounds__(256) void bias_cols_kernel(float* __restrict__ c, u
     c[i] = apply_epilogue(epi, i, c[i]);
 }
 
-// ---- split-K products folded inside the workgroup ----------------------------
-// A product whose plan splits K into S = 2..4 partitions (512^3: 4 of 4
-// K-tiles; a Linear(256, 100) layer at batch 128: 4 of 2) ran as the split
-// kernel writing S partial slices and split_k_reduce_kernel folding them: two
-// launches, the second bound by its launch and the partials' round trip
-// (10.4 us at 512^3 for 1.7 us of matrix-core work). Here a workgroup owns a
-// 32 x 32 output tile and one wave per partition: wave p stages its own
-// K-tiles [p*chunk, min((p+1)*chunk, ktiles)) in LDS (its K-slices of A and
-// B, zero outside the operands, with waits within the wave only) and runs the
-// 16 MFMA steps per K-tile that every kernel here runs (step t pairs k = t and
-// k = 16 + t), from 0, so its partial is the split kernel's. The S partials
-// then go through LDS and are folded per output exactly as the fold kernel
-// folds them (carry stack in partition order, drained from 0.0), with the
-// same epilogue: the product's bits, in one launch.
-constexpr int kWgFoldLdk = 33;  // LDS pitch of a staged 32 x 32 slice
+// ---- small products: one wave per partition, operands from registers -----------
+// A product whose 32x32 tiles and partitions fill no more than the card's
+// waves is bound by its chain of waits, not by the matrix cores: the split
+// kernel writing partial slices and the fold kernel reading them are two
+// launches (64x128x784: 5.6 + 2.8 us of kernels), and a one-tile product on the
+// LDS-staged tiles waits out load, store, barrier and read per K-tile (64x10x128
+// 9.6 us). Here a workgroup owns a 32x32 output tile and one wave per
+// partition. A wave reads its MFMA operands straight into registers, a lane its
+// row's 16 k of a 32-deep K-tile (lane half h: k = 16 h + 0..15; four 16-byte
+// loads at any float address for a k-contiguous operand, else 16 of 4 bytes),
+// two K-tiles ahead, and runs the 16 MFMA steps per K-tile that every fp32
+// kernel here runs (step t pairs k = t and k = 16 + t), from 0, so its partial
+// is the split kernel's. The partials meet in LDS and are folded per output
+// exactly as the fold kernel folds them (carry stack in partition order,
+// drained from 0.0), with the same epilogue: the plan's bits, in one launch.
+constexpr int kSmallMaxWaves = 8;  // small_fits
 
-template <int S, int KT>
-__global__ __launch_bounds__(64 * S) void gemm_wgfold_kernel(GemmArgs g, FoldEpilogue epi, int a_kfast,
-                                                             int b_kfast) {
-    // KT: K-tiles per partition, all of whose operand slices a wave loads
-    // into registers before its first MFMA (16-byte loads for a k-contiguous
-    // A and an n-contiguous B, the NN layout; elements otherwise)
-    __shared__ float stage[S][2][32 * kWgFoldLdk];  // per wave: A [row][k], B [col][k]
-    __shared__ float parts[S][16][64];
+// One operand's 16 values of K-tile kt for this lane: row (clamped by the
+// caller), k = 32 kt + 16 kh + 0..15, zero past K.
+__device__ __forceinline__ void small_load(float (&v)[16], const float* row, int64_t s_k, bool kfast, uint32_t k0,
+                                           uint32_t k) {
+    if (k0 + 16u <= k) {
+        if (kfast) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4u x = *reinterpret_cast<const f32x4u*>(row + k0 + 4 * q);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[4 * q + j] = x[j];
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) v[t] = row[static_cast<int64_t>(k0 + t) * s_k];
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const float x = row[static_cast<int64_t>(min(k0 + t, k - 1u)) * s_k];
+            v[t] = k0 + t < k ? x : 0.0f;
+        }
+    }
+}
+
+__global__ __launch_bounds__(64 * kSmallMaxWaves) void gemm_small_kernel(GemmArgs g, FoldEpilogue epi, uint32_t parts) {
+    extern __shared__ float partial[];  // [parts][16][64]
     const int lane = threadIdx.x & 63;
-    const int p = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint32_t p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lrow = lane & 31, kh = lane >> 5;
     const uint32_t tm = blockIdx.x / g.tiles_n, tn = blockIdx.x - tm * g.tiles_n;
     const uint32_t row0 = 32u * tm, col0 = 32u * tn;
     const uint32_t z = blockIdx.z;
     const uint32_t i0 = z / g.b1, i1 = z - i0 * g.b1;
-    const float* a = g.a + static_cast<int64_t>(i0) * g.sa0 + static_cast<int64_t>(i1) * g.sa1;
-    const float* b = g.b + static_cast<int64_t>(i0) * g.sb0 + static_cast<int64_t>(i1) * g.sb1;
-    float* As = stage[p][0];
-    float* Bs = stage[p][1];
-    const uint32_t kt0 = static_cast<uint32_t>(p) * g.chunk;
-    const uint32_t kt1 = min(g.ktiles, kt0 + g.chunk);
-    // the vector path: lane l loads row/k-row l/8 + 8q, 4 floats at 4*(l%8)
-    const bool vec = g.a_vec && g.b_vec && g.sak == 1 && g.sbn == 1;
-    float va[KT][16], vb[KT][16];
-#pragma unroll
-    for (int u = 0; u < KT; ++u) {
-        const uint32_t k0 = 32u * (kt0 + u);
-        const bool live = kt0 + u < kt1;
-        if (vec) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t rr = static_cast<uint32_t>(lane / 8 + 8 * q), c4 = 4u * (lane % 8);
-                const uint32_t gr = row0 + rr, gk = k0 + c4;
-                f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (live && gr < g.m && gk + 3 < g.k)
-                    x = *reinterpret_cast<const f32x4*>(a + static_cast<int64_t>(gr) * g.sam + gk);
-                else if (live && gr < g.m)
-                    for (int j = 0; j < 4; ++j)
-                        if (gk + j < g.k) x[j] = a[static_cast<int64_t>(gr) * g.sam + gk + j];
-                const uint32_t gbk = k0 + rr, gc = col0 + c4;
-                f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (live && gbk < g.k && gc + 3 < g.n)
-                    y = *reinterpret_cast<const f32x4*>(b + static_cast<int64_t>(gbk) * g.sbk + gc);
-                else if (live && gbk < g.k)
-                    for (int j = 0; j < 4; ++j)
-                        if (gc + j < g.n) y[j] = b[static_cast<int64_t>(gbk) * g.sbk + gc + j];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    va[u][4 * q + j] = x[j];
-                    vb[u][4 * q + j] = y[j];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t rr = a_kfast ? static_cast<uint32_t>(2 * i + kh) : static_cast<uint32_t>(lrow);
-                const uint32_t kk = a_kfast ? static_cast<uint32_t>(lrow) : static_cast<uint32_t>(2 * i + kh);
-                const uint32_t gr = row0 + rr, gk = k0 + kk;
-                va[u][i] = (live && gr < g.m && gk < g.k)
-                               ? a[static_cast<int64_t>(gr) * g.sam + static_cast<int64_t>(gk) * g.sak]
-                               : 0.0f;
-                const uint32_t cc = b_kfast ? static_cast<uint32_t>(2 * i + kh) : static_cast<uint32_t>(lrow);
-                const uint32_t bk = b_kfast ? static_cast<uint32_t>(lrow) : static_cast<uint32_t>(2 * i + kh);
-                const uint32_t gc = col0 + cc, gbk = k0 + bk;
-                vb[u][i] = (live && gc < g.n && gbk < g.k)
-                               ? b[static_cast<int64_t>(gbk) * g.sbk + static_cast<int64_t>(gc) * g.sbn]
-                               : 0.0f;
-            }
-        }
-    }
+    const float* a = g.a + static_cast<int64_t>(i0) * g.sa0 + static_cast<int64_t>(i1) * g.sa1 +
+                     static_cast<int64_t>(min(row0 + lrow, g.m - 1u)) * g.sam;
+    const float* b = g.b + static_cast<int64_t>(i0) * g.sb0 + static_cast<int64_t>(i1) * g.sb1 +
+                     static_cast<int64_t>(min(col0 + lrow, g.n - 1u)) * g.sbn;
+    const bool ak = g.sak == 1, bk = g.sbk == 1;
+    const uint32_t kt0 = p * g.chunk, kt1 = min(g.ktiles, kt0 + g.chunk);
+    float va[2][16], vb[2][16];
+    auto load = [&](int set, uint32_t kt) {
+        const uint32_t k0 = 32u * min(kt, kt1 - 1u) + 16u * kh;
+        small_load(va[set], a, g.sak, ak, k0, g.k);
+        small_load(vb[set], b, g.sbk, bk, k0, g.k);
+    };
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    load(0, kt0);
+    if (kt0 + 1 < kt1) load(1, kt0 + 1);
+    for (uint32_t kt = kt0; kt < kt1; kt += 2) {
 #pragma unroll
-    for (int u = 0; u < KT; ++u) {
-        if (kt0 + u >= kt1) break;
-        // (a wave's LDS operations complete in issue order; the fences keep
-        // the compiler from moving this K-tile's stores above the previous
-        // K-tile's reads, or its reads above these stores)
-        __builtin_amdgcn_wave_barrier();
-        asm volatile("" ::: "memory");
-        if (vec) {
+        for (int set = 0; set < 2; ++set) {
+            if (kt + set >= kt1) break;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int rr = lane / 8 + 8 * q, c = 4 * (lane % 8) + j;
-                    As[rr * kWgFoldLdk + c] = va[u][4 * q + j];  // A[row rr][k c]
-                    Bs[c * kWgFoldLdk + rr] = vb[u][4 * q + j];  // B[k rr][col c] as [col][k]
-                }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int rr = a_kfast ? 2 * i + kh : lrow, kk = a_kfast ? lrow : 2 * i + kh;
-                As[rr * kWgFoldLdk + kk] = va[u][i];
-                const int cc = b_kfast ? 2 * i + kh : lrow, bk = b_kfast ? lrow : 2 * i + kh;
-                Bs[cc * kWgFoldLdk + bk] = vb[u][i];
-            }
+            for (int t = 0; t < 16; ++t)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[set][t], vb[set][t], acc, 0, 0, 0);
+            if (kt + set + 2 < kt1) load(set, kt + set + 2);
         }
-        __builtin_amdgcn_wave_barrier();
-        asm volatile("" ::: "memory");
+    }
+    float* cz = g.c + static_cast<uint64_t>(z) * g.m * g.n;
+    auto store = [&](int r, int l, float v) {
+        const uint32_t row = row0 + 8 * (r / 4) + 4 * (l >> 5) + (r % 4), col = col0 + (l & 31);
+        if (row < g.m && col < g.n)
+            cz[static_cast<uint64_t>(row) * g.n + col] =
+                apply_epilogue(epi, (static_cast<uint64_t>(z) * g.m + row) * g.n + col, v);
+    };
+    if (parts == 1) {
 #pragma unroll
-        for (int t = 0; t < 16; ++t)
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[lrow * kWgFoldLdk + 16 * kh + t],
-                                                       Bs[lrow * kWgFoldLdk + 16 * kh + t], acc, 0, 0, 0);
+        for (int r = 0; r < 16; ++r) store(r, lane, acc[r]);
+        return;
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) parts[p][r][lane] = acc[r];
+    for (int r = 0; r < 16; ++r) partial[(p * 16 + r) * 64 + lane] = acc[r];
     __syncthreads();
-    // fold: output (r, l) of the tile, r = 0..15 register, l = lane
-    float* cz = g.c + static_cast<uint64_t>(z) * g.m * g.n;
-    for (int e = static_cast<int>(threadIdx.x); e < 1024; e += 64 * S) {
-        const int r = e >> 6, l = e & 63;
-        const uint32_t row = row0 + 8 * (r / 4) + 4 * (l >> 5) + (r % 4);
-        const uint32_t col = col0 + (l & 31);
+    for (uint32_t e = threadIdx.x; e < 1024; e += blockDim.x) {
         float stack[kSplitLevels];
 #pragma unroll
         for (int lv = 0; lv < kSplitLevels; ++lv) stack[lv] = 0.0f;
 #pragma unroll
-        for (int q = 0; q < S; ++q) carry_push(stack, static_cast<uint32_t>(q), parts[q][r][l]);
+        for (int q = 0; q < kSmallMaxWaves; ++q)
+            if (static_cast<uint32_t>(q) < parts) carry_push(stack, static_cast<uint32_t>(q), partial[q * 1024 + e]);
         float total = 0.0f;
 #pragma unroll
         for (int lv = 0; lv < kSplitLevels; ++lv)
-            if ((static_cast<uint32_t>(S) >> lv) & 1u) total = total + stack[lv];
-        if (row < g.m && col < g.n) {
-            const uint64_t i = (static_cast<uint64_t>(z) * g.m + row) * g.n + col;
-            cz[static_cast<uint64_t>(row) * g.n + col] = apply_epilogue(epi, i, total);
-        }
+            if ((parts >> lv) & 1u) total = total + stack[lv];
+        store(static_cast<int>(e >> 6), static_cast<int>(e & 63u), total);
     }
 }
 
@@ -2046,6 +2007,22 @@ struct TileChoice {
     uint64_t tiles = 0;     // output tiles of this tiling
     bool pair = false;      // partitions planned for pairs (two per workgroup)
 };
+
+// Whether a product with this plan runs on gemm_small_kernel. One CU does all
+// partitions of a 32x32 tile, 0.1 us of matrix core per K-tile, so the line is
+// the K-tiles a workgroup holds. Measured (us, NN / NT; the same launches as
+// two, or on 64x64 tiles): 4 partitions of 4 K-tiles 512^3 7.8 / 8.3 (8.6 /
+// 15.6), 333x777x211 8.7 / 8.7 (15.7 / 15.7), 8 of 2 100x1000x500 7.9 / 7.9
+// (9.0 / 8.8), 7 of 3 256x512x600 8.9 / 8.7 (9.9 / 9.9); not 13 of 2 64x128x784
+// 10.1 / 10.8 (7.1 / 6.9), 6 of 6 300x500x1000 13.8 / 13.4 (12.3 / 12.5).
+// Unsplit: 128x784x64 4.4 / 4.2 (4.8 / 4.7), 64x10x128 5.9 / 5.3 (6.6 / 5.6);
+// not 1024x1024x128 7.2 / 7.8 (6.5 / 6.4), whose 1024 waves of 4 K-tiles do
+// better sharing their operands through LDS.
+static bool small_fits(uint32_t batch, uint32_t m, uint32_t n, uint32_t splits, uint32_t chunk, const TileChoice& tile) {
+    const uint64_t t32 = static_cast<uint64_t>(ceil_div(m, 32u)) * ceil_div(n, 32u) * batch;
+    if (splits > 1) return !tile.pair && splits <= 8 && chunk <= 4 && splits * chunk <= 24;
+    return (chunk <= 2 && t32 <= 256) || (chunk <= 4 && t32 <= 8);
+}
 
 template <int BM, int BN, int WM, int WN, int AM>
 static void launch_b(const GemmArgs& g, dim3 grid, hipStream_t st, int bmode) {
@@ -2717,34 +2694,15 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
     // for a single pair); every other kernel one per partition.
     const bool direct128 = tile.bm == 128 && b_rows && (amode == KCD || a_rows);
     const bool paired = direct128 && tile.pair && splits >= 2 && reinterpret_cast<uintptr_t>(c) % 16 == 0;
-    // Two to four partitions on 64x64 tiles: one launch, the partials folded
-    // inside the workgroup (gemm_wgfold_kernel), the same bits; for products
-    // of at least 64 tiles of 32x32 (512^3: 256). Fewer tiles leave most CUs
-    // idle: the 128 x 100 x 256 product of a Linear(256, 100) layer (16
-    // tiles) took 10.3 us this way against 4.9 + 4.6 us as two launches.
-    const uint64_t t32_all = static_cast<uint64_t>(ceil_div(m, 32u)) * ceil_div(n, 32u) * batch;
-    if (splits >= 2 && splits <= 4 && chunk <= 4 && tile.bm == 64 && !tile.pair && t32_all >= 64) {
+    if (split_req == 0 && small_fits(static_cast<uint32_t>(batch), m, n, splits, chunk, tile)) {
         g.tiles_m = ceil_div(m, 32u);
         g.tiles_n = ceil_div(n, 32u);
-        const uint64_t t32 = static_cast<uint64_t>(g.tiles_m) * g.tiles_n;
-        if (t32 <= 0x7fffffffull) {
-            g.c = c;
-            const int akf = g.sak == 1 || g.sam != 1;
-            const int bkf = g.sbk == 1 || g.sbn != 1;
-            const dim3 grid(static_cast<uint32_t>(t32), 1, static_cast<uint32_t>(batch));
-#define VKHIP_WGF(SS, KT) \
-    hipLaunchKernelGGL((gemm_wgfold_kernel<SS, KT>), grid, dim3(64 * SS), 0, ctx().stream, g, fe, akf, bkf)
-#define VKHIP_WGF_S(KT) \
-    do { if (splits == 2) VKHIP_WGF(2, KT); else if (splits == 3) VKHIP_WGF(3, KT); else VKHIP_WGF(4, KT); } while (0)
-            if (chunk <= 2) VKHIP_WGF_S(2); else VKHIP_WGF_S(4);
-#undef VKHIP_WGF_S
-#undef VKHIP_WGF
-            VKHIP_LAUNCH_CHECK();
-            *fused = true;
-            return VKHIP_OK;
-        }
-        g.tiles_m = ceil_div(m, tile.bm);
-        g.tiles_n = ceil_div(n, tile.bn);
+        g.c = c;
+        hipLaunchKernelGGL(gemm_small_kernel, dim3(g.tiles_m * g.tiles_n, 1, static_cast<uint32_t>(batch)),
+                           dim3(64 * splits), splits > 1 ? splits * 4096u : 0u, ctx().stream, g, fe, splits);
+        VKHIP_LAUNCH_CHECK();
+        *fused = true;
+        return VKHIP_OK;
     }
     // Two partitions of a 64x64 tile grid that is one round of one workgroup
     // per CU: both in one workgroup, folded there (gemm_pair64_kernel).
