@@ -153,10 +153,11 @@ class DeviceArray:
 
     def is_contiguous(self) -> bool:
         expect = 1
-        for e, s in zip(reversed(self.shape), reversed(self.strides)):
+        for i in range(len(self.shape) - 1, -1, -1):
+            e = self.shape[i]
             if e == 1:
                 continue
-            if s != expect:
+            if self.strides[i] != expect:
                 return False
             expect *= e
         return True

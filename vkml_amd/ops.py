@@ -13,7 +13,7 @@ shape, error behaviour) and calls the matching C entry point of libvkhip:
 """
 from __future__ import annotations
 
-from ctypes import byref, c_uint32, c_void_p
+from ctypes import byref, c_uint32
 from typing import Iterable, Sequence
 
 import numpy as np
@@ -63,22 +63,25 @@ def matmul(a: DeviceArray, b: DeviceArray, *, kernel: int = _lib.GEMM_AUTO,
     if b.ndim == 1:
         b = DeviceArray((b.shape[0], 1), b.dtype, (b.strides[0], 0), b.buffer, b.offset)
         drop_n = True
-    if a.shape[-1] != b.shape[-2]:
+    m, k = a.shape[-2:]
+    if k != b.shape[-2]:
         raise ValueError(f"matmul inner dimensions disagree: {a.shape} @ {b.shape}")
-    batch = np.broadcast_shapes(a.shape[:-2], b.shape[:-2])
+    n = b.shape[-1]
+    ab, bb, batch = a, b, a.shape[:-2]
+    if batch != b.shape[:-2]:
+        batch = np.broadcast_shapes(batch, b.shape[:-2])
+        ab = a.broadcast_to(batch + (m, k))
+        bb = b.broadcast_to(batch + (k, n))
     if len(batch) > 2:
         raise ValueError("matmul supports at most two batch axes (rank 4)")
-    m, k, n = a.shape[-2], a.shape[-1], b.shape[-1]
-    ab = a.broadcast_to(batch + (m, k))
-    bb = b.broadcast_to(batch + (k, n))
     shape = batch + (m, n)
     if out is None:
         out = DeviceArray(shape, np.float32)
     elif out.shape != shape or not out.is_contiguous():
         raise ValueError("matmul: out must be contiguous with the result shape")
     opts = _lib.GemmOpts(kernel, split_k)
-    check(_lib.load().vkhip_gemm(c_void_p(ab.ptr), byref(ab.operand()), c_void_p(bb.ptr),
-                                 byref(bb.operand()), c_void_p(out.ptr), byref(opts)), "matmul")
+    check(_lib.load().vkhip_gemm(ab.ptr, byref(ab.operand()), bb.ptr, byref(bb.operand()), out.ptr,
+                                 byref(opts)), "matmul")
     if drop_m or drop_n:
         final = list(shape)
         if drop_n:
@@ -96,17 +99,17 @@ def split_k_reduce(ws: DeviceArray, splits: int) -> DeviceArray:
         raise ValueError("split_k_reduce: workspace must be contiguous, splits * ne elements")
     ne = ws.size // splits
     out = DeviceArray((ne,), np.float32)
-    check(_lib.load().vkhip_split_k_reduce(c_void_p(ws.ptr), c_void_p(out.ptr), ne, splits),
+    check(_lib.load().vkhip_split_k_reduce(ws.ptr, out.ptr, ne, splits),
           "split_k_reduce")
     return out
 
 
 def _out(out: DeviceArray | None, shape, dtype=np.float32) -> DeviceArray:
     """The result buffer: `out` if given (contiguous, right shape), else new."""
-    shape = tuple(int(e) for e in shape)
+    shape = tuple(shape)
     if out is None:
         return DeviceArray(shape, dtype)
-    if out.shape != shape or out.dtype != np.dtype(dtype) or not out.is_contiguous():
+    if out.shape != shape or out.dtype != dtype or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous {np.dtype(dtype)} array of shape {shape}")
     return out
 
@@ -118,8 +121,8 @@ def gemv(a: DeviceArray, x: DeviceArray, out: DeviceArray | None = None) -> Devi
     if a.ndim != 2 or x.ndim != 1 or a.shape[1] != x.shape[0] or a.strides[1] != 1:
         raise ValueError("gemv: expects A [M,K] with unit inner stride and x [K]")
     y = _out(out, (a.shape[0],))
-    check(_lib.load().vkhip_gemv(c_void_p(a.ptr), a.strides[0], c_void_p(x.ptr), x.strides[0],
-                                 c_void_p(y.ptr), a.shape[0], a.shape[1]), "gemv")
+    check(_lib.load().vkhip_gemv(a.ptr, a.strides[0], x.ptr, x.strides[0],
+                                 y.ptr, a.shape[0], a.shape[1]), "gemv")
     return y
 
 
@@ -146,7 +149,7 @@ def im2col(x: DeviceArray, kernel, stride=1, padding=0, dilation=1,
         raise ValueError("im2col: kernel larger than the padded image")
     out = _out(out, (n, c * kh * kw, oh * ow))
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (dh, dw), (h, w))
-    check(_lib.load().vkhip_im2col(c_void_p(x.ptr), byref(x.operand()), c_void_p(out.ptr),
+    check(_lib.load().vkhip_im2col(x.ptr, byref(x.operand()), out.ptr,
                                    byref(u)), "im2col")
     return out
 
@@ -173,7 +176,7 @@ def col2im(cols: DeviceArray, image_hw, kernel, stride=1, padding=0, dilation=1,
     c = rows // (kh * kw)
     out = _out(out, (n, c, h, w))
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (dh, dw), (h, w))
-    check(_lib.load().vkhip_col2im(c_void_p(cols.ptr), c_void_p(out.ptr), n, c, byref(u)),
+    check(_lib.load().vkhip_col2im(cols.ptr, out.ptr, n, c, byref(u)),
           "col2im")
     return out
 
@@ -205,8 +208,8 @@ def conv2d(x: DeviceArray, weight: DeviceArray, stride=1, padding=0, dilation=1,
     out = _out(out, (n, cout, oh, ow))
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (dh, dw), (h, w))
     wd = _lib.operand((cout, cin * kh * kw), (cin * kh * kw, 1))
-    check(_lib.load().vkhip_conv2d(c_void_p(x.ptr), byref(x.operand()), c_void_p(weight.ptr),
-                                   byref(wd), c_void_p(out.ptr), byref(u)), "conv2d")
+    check(_lib.load().vkhip_conv2d(x.ptr, byref(x.operand()), weight.ptr,
+                                   byref(wd), out.ptr, byref(u)), "conv2d")
     return out
 
 
@@ -235,8 +238,8 @@ def conv2d_weight_grad(x: DeviceArray, grad: DeviceArray, kernel, stride=1, padd
     out = _out(out, (n, cout, c * kh * kw))
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (dh, dw), (h, w))
     gd = _lib.operand((1, n, cout, oh * ow), (0, cout * oh * ow, oh * ow, 1))
-    check(_lib.load().vkhip_conv2d_weight_grad(c_void_p(x.ptr), byref(x.operand()),
-                                               c_void_p(grad.ptr), byref(gd), c_void_p(out.ptr),
+    check(_lib.load().vkhip_conv2d_weight_grad(x.ptr, byref(x.operand()),
+                                               grad.ptr, byref(gd), out.ptr,
                                                byref(u)), "conv2d_weight_grad")
     return out
 
@@ -270,8 +273,8 @@ def conv2d_input_grad(grad: DeviceArray, weight: DeviceArray, image_hw, stride=1
     out = _out(out, (n, c, h, w))
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (dh, dw), (h, w))
     wd = _lib.operand((1, 1, cout, c * kh * kw), (0, 0, c * kh * kw, 1))
-    check(_lib.load().vkhip_conv2d_input_grad(c_void_p(grad.ptr), byref(grad.operand()),
-                                              c_void_p(weight.ptr), byref(wd), c_void_p(out.ptr),
+    check(_lib.load().vkhip_conv2d_input_grad(grad.ptr, byref(grad.operand()),
+                                              weight.ptr, byref(wd), out.ptr,
                                               byref(u)), "conv2d_input_grad")
     return out
 
@@ -303,8 +306,8 @@ def conv2d_weight_grad_sum(x: DeviceArray, grad: DeviceArray, kernel, stride=1, 
     out = _out(out, (cout, c * kh * kw))
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (dh, dw), (h, w))
     gd = _lib.operand((1, n, cout, oh * ow), (0, cout * oh * ow, oh * ow, 1))
-    check(_lib.load().vkhip_conv2d_weight_grad_sum(c_void_p(x.ptr), byref(x.operand()),
-                                                   c_void_p(grad.ptr), byref(gd), c_void_p(out.ptr),
+    check(_lib.load().vkhip_conv2d_weight_grad_sum(x.ptr, byref(x.operand()),
+                                                   grad.ptr, byref(gd), out.ptr,
                                                    byref(u)), "conv2d_weight_grad_sum")
     return out
 
@@ -321,7 +324,7 @@ def softmax(x: DeviceArray, axis: int = -1, log: bool = False,
             out: DeviceArray | None = None) -> DeviceArray:
     _f32(x, "softmax")
     out = _out(out, x.shape)
-    check(_lib.load().vkhip_softmax(c_void_p(x.ptr), byref(x.operand()), c_void_p(out.ptr),
+    check(_lib.load().vkhip_softmax(x.ptr, byref(x.operand()), out.ptr,
                                     _axis4(x, axis), 1 if log else 0), "softmax")
     return out
 
@@ -345,8 +348,8 @@ def _reduce(op: int, x: DeviceArray, axes, keepdim: bool,
     shape = [1 if i in axes else e for i, e in enumerate(x.shape)] if keepdim else kept
     dt = np.int64 if op in (_lib.REDUCE_ARGMAX, _lib.REDUCE_ARGMIN) else np.float32
     out = _out(out, shape, dt)
-    check(_lib.load().vkhip_reduce(op, c_void_p(x.ptr), byref(x.operand()), mask,
-                                   c_void_p(out.ptr)), "reduce")
+    check(_lib.load().vkhip_reduce(op, x.ptr, byref(x.operand()), mask,
+                                   out.ptr), "reduce")
     return out
 
 
@@ -395,7 +398,7 @@ def max_pool2d(x: DeviceArray, kernel, stride=None, padding=0) -> DeviceArray:
     oh, ow = window_count(h, kh, sh, ph, 1), window_count(w, kw, sw, pw, 1)
     out = DeviceArray((n, c, oh, ow), np.float32)
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (1, 1), (h, w))
-    check(_lib.load().vkhip_max_pool2d(c_void_p(x.ptr), c_void_p(out.ptr), n * c, oh, ow,
+    check(_lib.load().vkhip_max_pool2d(x.ptr, out.ptr, n * c, oh, ow,
                                        byref(u)), "max_pool2d")
     return out
 
@@ -414,8 +417,8 @@ def max_pool2d_backward(grad: DeviceArray, x: DeviceArray, kernel, stride=None,
     n, c, h, w = x.shape
     out = DeviceArray(x.shape, np.float32)
     u = _lib.unfold((kh, kw), (sh, sw), (ph, pw), (1, 1), (h, w))
-    check(_lib.load().vkhip_max_pool2d_backward(c_void_p(grad.ptr), c_void_p(x.ptr),
-                                                c_void_p(out.ptr), n * c, grad.shape[2],
+    check(_lib.load().vkhip_max_pool2d_backward(grad.ptr, x.ptr,
+                                                out.ptr, n * c, grad.shape[2],
                                                 grad.shape[3], byref(u)), "max_pool2d_backward")
     return out
 
@@ -425,7 +428,7 @@ def scaled_add(a: DeviceArray, b: DeviceArray, alpha: float, beta: float) -> Dev
     if a.shape != b.shape or not (a.is_contiguous() and b.is_contiguous()):
         raise ValueError("scaled_add: contiguous operands of one shape")
     out = DeviceArray(a.shape, np.float32)
-    check(_lib.load().vkhip_scaled_add(c_void_p(a.ptr), c_void_p(b.ptr), c_void_p(out.ptr),
+    check(_lib.load().vkhip_scaled_add(a.ptr, b.ptr, out.ptr,
                                        a.size, alpha, beta), "scaled_add")
     return out
 
