@@ -2318,6 +2318,15 @@ static double triple_time(const TripleTileTimes& t, uint64_t tiles, uint32_t sli
 // 11.4 and 12.6; above, 700^3 17.1 and 16.4, 1024^3 24.7 and 20.7.
 constexpr double kTripleMinMacs = 268435456.0;
 
+// Not for a launch that leaves half of the CUs idle (a batch, whose images are
+// not split): a convolution's workgroups there wait for their own gathers,
+// [32,96,16,16] -> 64 3x3 22.8 us on the fp32 cores and 25.5 here, [16,128,16,16]
+// -> 128 25.9 and 30.7, its columns as a product 24.4 and 22.3. Nor for one row
+// of tiles over a short K, whose epilogue weighs as much: [64,32,28,28] -> 64
+// 3x3 27.1 and 28.7 ([32,64,16,16] -> 128 3x3, twice the K, 21.0 and 18.9);
+// nor for batches of tall shallow products, the columns of a strided input
+// gradient, all output: [20,96,32,32] -> 96 3x3 stride 2 (20 of 864x256x96)
+// 38.9 and 45.1, [64,64,32,32] -> 128 (64 of 576x256x128) 67.3 and 73.8.
 static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
     TriplePlan best;
     if (m <= 32 || n <= 32 || k < 64) return best;
@@ -2350,6 +2359,9 @@ static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k
             }
         }
     }
+    const TripleTileTimes& tt = kTripleTiles[best.tile];
+    const uint64_t wgs = static_cast<uint64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch * best.slices;
+    if (2.0 * wgs <= cus || (std::min(m, n) <= 64 && k <= 320) || (batch > 1 && m > 128 && k <= 128)) return TriplePlan{};
     return best;
 }
 
@@ -4037,7 +4049,14 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     const int amode = g.a_vec ? KCV : KCS;
     const uint64_t out_elems = static_cast<uint64_t>(m) * n;
     float* target = out;
-    const TriplePlan triple = g.sa1 >= 0 && triple_mode(m, static_cast<uint32_t>(L), g.sam, g.sak) == TK &&
+    // Where 32-deep K-tiles stay inside an image the fp32 kernels are ahead of
+    // the three terms, which gather and split the columns once per row of tiles
+    // ([48,64,16,16] -> 128 3x3 44.9 us against 49.1, [32,64,32,32] -> 64 55.2
+    // and 61.3, [24,96,16,16] -> 96 37.0 and 40.9); where they cross images
+    // behind ([64,32,28,28] -> 64 3x3 54.2 and 37.1, [32,128,14,14] -> 96 41.1
+    // and 36.4).
+    const TriplePlan triple = L % 32 != 0 && g.sa1 >= 0 &&
+                                      triple_mode(m, static_cast<uint32_t>(L), g.sam, g.sak) == TK &&
                                       triple_image_fits(im, oh)
                                   ? triple_plan(1, m, n, k) : TriplePlan{};
     if (triple) splits = triple.slices;
