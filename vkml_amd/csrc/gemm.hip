@@ -4054,8 +4054,10 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     // ([48,64,16,16] -> 128 3x3 44.9 us against 49.1, [32,64,32,32] -> 64 55.2
     // and 61.3, [24,96,16,16] -> 96 37.0 and 40.9); where they cross images
     // behind ([64,32,28,28] -> 64 3x3 54.2 and 37.1, [32,128,14,14] -> 96 41.1
-    // and 36.4).
-    const TriplePlan triple = L % 32 != 0 && g.sa1 >= 0 &&
+    // and 36.4), and where two rows of tiles share a gather over a deep K
+    // (K 32768, [128,64,16,16] -> 128 3x3 63.6 and 55.3, and 65536, [64,128,32,32] -> 128 1x1
+    // 42.5 and 33.6; K 12288 is the 44.9 against 49.1 above).
+    const TriplePlan triple = (L % 32 != 0 || (std::min(m, n) > 64 && k >= 32768)) && g.sa1 >= 0 &&
                                       triple_mode(m, static_cast<uint32_t>(L), g.sam, g.sak) == TK &&
                                       triple_image_fits(im, oh)
                                   ? triple_plan(1, m, n, k) : TriplePlan{};
