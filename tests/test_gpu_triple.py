@@ -7,7 +7,8 @@ import pytest
 
 from conftest import SEED, gemm_tolerance, normwise_rel_err
 from vkml_amd import ops
-from vkml_amd.device import DeviceArray
+from vkml_amd import tensor as T
+from vkml_amd.device import DeviceArray, DecisionRecorder
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +117,35 @@ def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stri
     exact = np.einsum("nol,nkl->ok", g.reshape(n, cout, L).astype(np.float64), cols.numpy().astype(np.float64),
                       optimize=True)
     assert normwise_rel_err(total, exact) <= 2.0 ** -23 * np.sqrt(n * L)
+
+
+def _operand_kinds(rec: DecisionRecorder) -> list[str]:
+    return [d["chose"] for d in rec.decisions if d["site"] == "matmul.operands"]
+
+
+def test_graph_nodes_keep_the_fp32_kernels(hip):
+    """Products and convolutions of a graph, forward and backward, have the
+    bits of the fp32 kernels: another order of sums moves a near tie of a
+    pool or relu, and the gradients behind it by far more than rounding."""
+    rng = np.random.default_rng(SEED + 3)
+    x = rng.uniform(-1, 1, (96, 64, 16, 16)).astype(np.float32)
+    w = rng.uniform(-0.05, 0.05, (128, 64, 3, 3)).astype(np.float32)
+    u, v = rng.standard_normal((1000, 777)).astype(np.float32), rng.standard_normal((1501, 777)).astype(np.float32)
+    with DecisionRecorder() as rec:
+        tx, tw = T.tensor(x, requires_grad=True), T.tensor(w, requires_grad=True)
+        y = T.conv2d(tx, tw, padding=1)
+        T.backward(T.sum(y))
+        tu, tv = T.tensor(u, requires_grad=True), T.tensor(v, requires_grad=True)
+        z = T.matmul(tu, tv.transpose(-2, -1))
+        T.backward(T.sum(z))
+        got = [t.numpy() for t in (y, tx.grad, tw.grad, z, tu.grad, tv.grad)]
+    assert _operand_kinds(rec) == []
+    # plans of one partition: split_k=1 is the fp32 kernel of the same plan
+    assert ops.gemm_plan(96, 128, 256, 576)[0] == ops.gemm_plan(1, 1000, 1501, 777)[0] == 1
+    cols = ops.im2col(DeviceArray.from_numpy(x), 3, 1, 1).reshape(1, 96, 576, 256)
+    flat = DeviceArray.from_numpy(w.reshape(1, 1, 128, 576)).broadcast_to((1, 96, 128, 576))
+    assert np.array_equal(got[0].reshape(-1), ops.matmul(flat, cols, split_k=1).numpy().reshape(-1))
+    assert np.array_equal(got[3], ops.matmul(_view(u, "n"), _view(v, "n").T, split_k=1).numpy())
+    ones = np.ones((1000, 1501))
+    for grad, exact in ((got[4], ones @ v), (got[5], ones.T @ u)):
+        assert normwise_rel_err(grad, exact) <= gemm_tolerance(1501)

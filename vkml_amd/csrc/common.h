@@ -100,9 +100,14 @@ struct GemmEpilogue {
     bool relu;
     const float* mask = nullptr;
 };
+// terms: a product may run as bf16 terms (gemm_triple.h). Only the per-op
+// entry points allow it; a node's values go on into comparisons (a pool
+// window's maximum, a relu's zero), where another order of sums moves a near
+// tie and with it a gradient by 4e-3 of its norm (the two-convolution network
+// at batch 128), so nodes keep the order of the fp32 kernels.
 int gemm(const float* a, const vkhip_operand& ad, const float* b, const vkhip_operand& bd, float* c,
          const vkhip_gemm_opts* opts, const FixedScratch* scratch = nullptr,
-         const GemmEpilogue* epi = nullptr);
+         const GemmEpilogue* epi = nullptr, bool terms = false);
 
 // Decision facts and units of work (observe.hip). A unit is a node of
 // vkhip_compute or one per-op entry call; decisions published inside it carry

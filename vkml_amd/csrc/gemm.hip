@@ -2553,7 +2553,7 @@ static double round_fill(uint64_t wgs, uint64_t slots) {
 
 static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, const vkhip_operand& bd,
                      float* c, const vkhip_gemm_opts* opts, const FixedScratch* scratch,
-                     const FoldEpilogue& fe, bool* fused) {
+                     const FoldEpilogue& fe, bool* fused, bool terms) {
     const uint32_t b0 = ad.ne[0] > bd.ne[0] ? ad.ne[0] : bd.ne[0];
     const uint32_t b1 = ad.ne[1] > bd.ne[1] ? ad.ne[1] : bd.ne[1];
     const uint32_t m = ad.ne[2], k = ad.ne[3], n = bd.ne[3];
@@ -2655,7 +2655,7 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
                   : (g.sbn == 1 && aligned(b, g.sb0, g.sb1, g.sbk));
 
     const uint64_t out_elems = batch * m * n;
-    if (split_req == 0) {
+    if (terms && split_req == 0) {
         const TriplePlan t = triple_plan(static_cast<uint32_t>(batch), m, n, k);
         if (t) {
             publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, t.chunk, t.slices);
@@ -2838,10 +2838,10 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
 }
 
 int gemm(const float* a, const vkhip_operand& ad, const float* b, const vkhip_operand& bd, float* c,
-         const vkhip_gemm_opts* opts, const FixedScratch* scratch, const GemmEpilogue* epi) {
+         const vkhip_gemm_opts* opts, const FixedScratch* scratch, const GemmEpilogue* epi, bool terms) {
     const FoldEpilogue fe = fold_epilogue(epi, bd.ne[3]);
     bool fused = false;
-    const int st = gemm_core(a, ad, b, bd, c, opts, scratch, fe, &fused);
+    const int st = gemm_core(a, ad, b, bd, c, opts, scratch, fe, &fused, terms);
     if (st != VKHIP_OK || (!fe.bias && !fe.mask) || fused) return st;
     // no split (or the GEMV, the exact arm, K == 0): the epilogue as a pass
     const uint64_t rows = static_cast<uint64_t>(std::max(ad.ne[0], bd.ne[0])) *
@@ -3503,7 +3503,7 @@ static int launch_conv_wgrad_stream(SmallConvFwd p, const float* gr, const vkhip
 
 int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
                    const vkhip_operand& wd, float* out, const vkhip_unfold& p, const float* bias,
-                   int64_t bias_stride, bool relu) {
+                   int64_t bias_stride, bool relu, bool terms) {
     if (p.kernel_h <= 0 || p.kernel_w <= 0 || p.stride_h <= 0 || p.stride_w <= 0 ||
         p.dilation_h <= 0 || p.dilation_w <= 0 || p.pad_h < 0 || p.pad_w < 0)
         return fail(VKHIP_ERR_INVALID, "conv2d: invalid window geometry");
@@ -3605,7 +3605,7 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     const uint64_t out_elems = batch * m * n;
     float* target = out;
     // the plan gemm() takes for the same product, so the same bits
-    const TriplePlan triple = triple_mode(m, k, g.sam, g.sak) == TK
+    const TriplePlan triple = terms && triple_mode(m, k, g.sam, g.sak) == TK
                                   ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
     if (triple) splits = triple.slices;
     if (splits > 1) {
@@ -3686,7 +3686,7 @@ static bool wgrad_direct_fits(const GemmArgs& g, uint32_t positions, const float
 }
 
 int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
-                       const vkhip_operand& gd, float* out, const vkhip_unfold& p) {
+                       const vkhip_operand& gd, float* out, const vkhip_unfold& p, bool terms) {
     if (static_cast<int64_t>(xd.ne[2]) != p.image_h || static_cast<int64_t>(xd.ne[3]) != p.image_w)
         return fail(VKHIP_ERR_INVALID, "conv2d weight grad: image is %ux%u but the geometry says %dx%d",
                     xd.ne[2], xd.ne[3], p.image_h, p.image_w);
@@ -3775,7 +3775,7 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     const int amode = a_kcd ? KCD : (g.a_vec ? KCV : KCS);
     const uint64_t out_elems = batch * m * n;
     float* target = out;
-    const TriplePlan triple = g.sa1 >= 0 && triple_mode(m, k, g.sam, g.sak) == TK && triple_image_fits(im, oh)
+    const TriplePlan triple = terms && g.sa1 >= 0 && triple_mode(m, k, g.sam, g.sak) == TK && triple_image_fits(im, oh)
                                   ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
     if (triple) splits = triple.slices;
     if (splits > 1) {
@@ -3820,7 +3820,7 @@ int launch_col2im(const float* cols, float* dst, uint32_t n, uint32_t channels, 
 int launch_max_pool2d_backward(const float* grad, const float* src, const vkhip_operand& sd, float* dst,
                                uint32_t out_h, uint32_t out_w, const vkhip_unfold& p, bool relu);
 int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float* gr, const vkhip_operand& gd,
-                           float* out, const vkhip_unfold& p);
+                           float* out, const vkhip_unfold& p, bool terms);
 
 // The weight and bias gradients of a conv layer whose output y = relu(conv2d(x,
 // w) + bias) feeds a 2x2, stride-2 max-pool, from the pool's output gradient gp
@@ -3887,7 +3887,7 @@ int conv2d_pool_weight_bias_grad(const float* x, const vkhip_operand& xd, const 
     dgd.nb[1] = static_cast<int64_t>(cout) * static_cast<int64_t>(L);
     dgd.nb[2] = static_cast<int64_t>(L);
     dgd.nb[3] = 1;
-    st = conv2d_weight_grad_sum(x, xd, dz, dgd, out, p);
+    st = conv2d_weight_grad_sum(x, xd, dz, dgd, out, p, false);
     if (st != VKHIP_OK) return st;
     vkhip_operand rd;  // dz [N, Cout, oh, ow], summed over axes 0, 2, 3
     rd.ne[0] = batch;
@@ -3915,7 +3915,7 @@ int conv2d_pool_weight_bias_grad(const float* x, const vkhip_operand& xd, const 
 //    (conv2d_weight_grad, exact in the exact mode) into a node temporary,
 //    then the batch sum's pairwise reduction: the graph's bits.
 int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float* gr,
-                           const vkhip_operand& gd, float* out, const vkhip_unfold& p) {
+                           const vkhip_operand& gd, float* out, const vkhip_unfold& p, bool terms) {
     if (static_cast<int64_t>(xd.ne[2]) != p.image_h || static_cast<int64_t>(xd.ne[3]) != p.image_w)
         return fail(VKHIP_ERR_INVALID, "conv2d weight grad sum: image is %ux%u but the geometry says %dx%d",
                     xd.ne[2], xd.ne[3], p.image_h, p.image_w);
@@ -3945,7 +3945,7 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
         const uint64_t per = static_cast<uint64_t>(cout) * ck;
         int st = node_temporary(batch * per * sizeof(float), &tmp);
         if (st != VKHIP_OK) return st;
-        st = conv2d_weight_grad(x, xd, gr, gd, tmp, p);
+        st = conv2d_weight_grad(x, xd, gr, gd, tmp, p, terms);
         if (st != VKHIP_OK) return st;
         vkhip_operand td;
         td.ne[0] = 1;
@@ -4057,7 +4057,7 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     // and 36.4), and where two rows of tiles share a gather over a deep K
     // (K 32768, [128,64,16,16] -> 128 3x3 63.6 and 55.3, and 65536, [64,128,32,32] -> 128 1x1
     // 42.5 and 33.6; K 12288 is the 44.9 against 49.1 above).
-    const TriplePlan triple = (L % 32 != 0 || (std::min(m, n) > 64 && k >= 32768)) && g.sa1 >= 0 &&
+    const TriplePlan triple = terms && (L % 32 != 0 || (std::min(m, n) > 64 && k >= 32768)) && g.sa1 >= 0 &&
                                       triple_mode(m, static_cast<uint32_t>(L), g.sam, g.sak) == TK &&
                                       triple_image_fits(im, oh)
                                   ? triple_plan(1, m, n, k) : TriplePlan{};
@@ -4125,7 +4125,7 @@ __global__ void conv_weight_flip_kernel(const float* __restrict__ w, int64_t s_o
 // K = Cout*kh*kw). Exact numerics, other strides or pad > dilation*(k-1) run
 // the graph: the TN product into a column matrix, then col2im.
 int conv2d_input_grad(const float* gr, const vkhip_operand& gd, const float* w, int64_t w_row,
-                      uint32_t channels, float* out, const vkhip_unfold& p) {
+                      uint32_t channels, float* out, const vkhip_unfold& p, bool terms) {
     if (p.kernel_h <= 0 || p.kernel_w <= 0 || p.stride_h <= 0 || p.stride_w <= 0 ||
         p.dilation_h <= 0 || p.dilation_w <= 0 || p.pad_h < 0 || p.pad_w < 0 || p.image_h < 0 ||
         p.image_w < 0)
@@ -4198,7 +4198,7 @@ int conv2d_input_grad(const float* gr, const vkhip_operand& gd, const float* w, 
         wd.nb[1] = 0;
         wd.nb[2] = static_cast<int64_t>(cout) * kk;
         wd.nb[3] = 1;
-        return conv2d_forward(gr, gd, wt, wd, out, q, nullptr, 0, false);
+        return conv2d_forward(gr, gd, wt, wd, out, q, nullptr, 0, false, terms);
     }
     if (ck > 0xffffffffull || L > 0xffffffffull)
         return fail(VKHIP_ERR_UNSUPPORTED, "conv2d input grad: extents too large");
@@ -4224,7 +4224,7 @@ int conv2d_input_grad(const float* gr, const vkhip_operand& gd, const float* w, 
     bd.nb[2] = gd.nb[1];
     bd.nb[3] = 1;
     const vkhip_gemm_opts opts{ctx().node_gemm_kernel, 0};
-    st = gemm(w, ad, gr, bd, cols, &opts);
+    st = gemm(w, ad, gr, bd, cols, &opts, nullptr, nullptr, terms);
     if (st != VKHIP_OK) return st;
     return launch_col2im(cols, out, batch, channels, p);
 }
@@ -4237,7 +4237,7 @@ extern "C" int vkhip_gemm(const float* a, const vkhip_operand* a_desc, const flo
     if (st != VKHIP_OK) return st;
     vkhip::Unit unit("matmul");
     if (!a_desc || !b_desc) return vkhip::fail(VKHIP_ERR_INVALID, "gemm: null descriptor");
-    return vkhip::gemm(a, *a_desc, b, *b_desc, c, opts);
+    return vkhip::gemm(a, *a_desc, b, *b_desc, c, opts, nullptr, nullptr, true);
 }
 
 extern "C" int vkhip_gemm_noalloc(const float* a, const vkhip_operand* a_desc, const float* b,
@@ -4250,7 +4250,7 @@ extern "C" int vkhip_gemm_noalloc(const float* a, const vkhip_operand* a_desc, c
         return vkhip::fail(VKHIP_ERR_UNSUPPORTED, "gemm_noalloc: no scratch array on device %d",
                            vkhip::ctx().device);
     const vkhip::FixedScratch fixed{vkhip::ctx().scratch, VKHIP_GEMM_NOALLOC_SCRATCH_BYTES};
-    return vkhip::gemm(a, *a_desc, b, *b_desc, c, opts, &fixed);
+    return vkhip::gemm(a, *a_desc, b, *b_desc, c, opts, &fixed, nullptr, true);
 }
 
 extern "C" int vkhip_gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k,
@@ -4295,7 +4295,7 @@ extern "C" int vkhip_conv2d(const float* x, const vkhip_operand* x_desc, const f
     if (st != VKHIP_OK) return st;
     vkhip::Unit unit("conv2d");
     if (!x_desc || !w_desc || !p) return vkhip::fail(VKHIP_ERR_INVALID, "conv2d: null argument");
-    return vkhip::conv2d_forward(x, *x_desc, w, *w_desc, out, *p, nullptr, 0, false);
+    return vkhip::conv2d_forward(x, *x_desc, w, *w_desc, out, *p, nullptr, 0, false, true);
 }
 
 extern "C" int vkhip_conv2d_weight_grad(const float* x, const vkhip_operand* x_desc,
@@ -4305,7 +4305,7 @@ extern "C" int vkhip_conv2d_weight_grad(const float* x, const vkhip_operand* x_d
     if (st != VKHIP_OK) return st;
     vkhip::Unit unit("conv2d_weight_grad");
     if (!x_desc || !grad_desc || !p) return vkhip::fail(VKHIP_ERR_INVALID, "conv2d weight grad: null argument");
-    return vkhip::conv2d_weight_grad(x, *x_desc, grad, *grad_desc, out, *p);
+    return vkhip::conv2d_weight_grad(x, *x_desc, grad, *grad_desc, out, *p, true);
 }
 
 extern "C" int vkhip_conv2d_input_grad(const float* grad, const vkhip_operand* grad_desc,
@@ -4321,7 +4321,7 @@ extern "C" int vkhip_conv2d_input_grad(const float* grad, const vkhip_operand* g
         return vkhip::fail(VKHIP_ERR_INVALID,
                            "conv2d_input_grad: weight must be [1,1,Cout,C*kh*kw] with contiguous rows");
     return vkhip::conv2d_input_grad(grad, *grad_desc, w, w_desc->nb[2],
-                                    static_cast<uint32_t>(w_desc->ne[3] / kk), out, *p);
+                                    static_cast<uint32_t>(w_desc->ne[3] / kk), out, *p, true);
 }
 
 extern "C" int vkhip_conv2d_weight_grad_sum(const float* x, const vkhip_operand* x_desc,
@@ -4331,7 +4331,7 @@ extern "C" int vkhip_conv2d_weight_grad_sum(const float* x, const vkhip_operand*
     if (st != VKHIP_OK) return st;
     vkhip::Unit unit("conv2d_weight_grad_sum");
     if (!x_desc || !grad_desc || !p) return vkhip::fail(VKHIP_ERR_INVALID, "conv2d_weight_grad_sum: null argument");
-    return vkhip::conv2d_weight_grad_sum(x, *x_desc, grad, *grad_desc, out, *p);
+    return vkhip::conv2d_weight_grad_sum(x, *x_desc, grad, *grad_desc, out, *p, true);
 }
 
 extern "C" uint32_t vkhip_kcd_slot_offset(uint32_t slot, int64_t s_row, uint32_t row0, uint32_t rows,

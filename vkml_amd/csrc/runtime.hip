@@ -20,19 +20,20 @@ namespace vkhip {
 int launch_im2col(const float* src, const vkhip_operand& sd, float* dst, const vkhip_unfold& p);
 int launch_col2im(const float* cols, float* dst, uint32_t n, uint32_t channels,
                   const vkhip_unfold& p);
+// (terms: as gemm()'s; a node passes false)
 int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
                    const vkhip_operand& wd, float* out, const vkhip_unfold& p, const float* bias,
-                   int64_t bias_stride, bool relu);
+                   int64_t bias_stride, bool relu, bool terms);
 int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
-                       const vkhip_operand& gd, float* out, const vkhip_unfold& p);
+                       const vkhip_operand& gd, float* out, const vkhip_unfold& p, bool terms);
 int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float* gr,
-                           const vkhip_operand& gd, float* out, const vkhip_unfold& p);
+                           const vkhip_operand& gd, float* out, const vkhip_unfold& p, bool terms);
 int launch_max_pool2x2_backward_relu_sums(const float* grad, const float* src, const vkhip_operand& sd,
                                           float* dst, float* bias_out);
 int conv2d_pool_weight_bias_grad(const float* x, const vkhip_operand& xd, const float* y, const vkhip_operand& yd,
                                  const float* gp, const vkhip_operand& gpd, float* out, const vkhip_unfold& p);
 int conv2d_input_grad(const float* gr, const vkhip_operand& gd, const float* w, int64_t w_row,
-                      uint32_t channels, float* out, const vkhip_unfold& p);
+                      uint32_t channels, float* out, const vkhip_unfold& p, bool terms);
 int launch_cross_entropy(const float* logits, int64_t row_stride, const int64_t* labels,
                          const float* g_out, float* out, uint32_t rows, uint32_t n, int backward);
 int launch_max_pool2d(const float* src, const vkhip_operand& sd, float* dst, uint32_t out_h,
@@ -726,7 +727,7 @@ static int compute_node(const vkhip_node& nd) {
                                   static_cast<const float*>(w.data), wd,
                                   static_cast<float*>(nd.out.data), p,
                                   fused ? static_cast<const float*>(nd.src[2].data) : nullptr,
-                                  fused ? nd.src[2].nb[0] : 0, fused);
+                                  fused ? nd.src[2].nb[0] : 0, fused, false);
         }
         case VKHIP_OP_CONV2D_WEIGHT_GRAD: {
             vkhip_unfold p;
@@ -749,7 +750,7 @@ static int compute_node(const vkhip_node& nd) {
             gd.nb[3] = 1;
             return conv2d_weight_grad(static_cast<const float*>(nd.src[0].data), to_operand(nd.src[0]),
                                       static_cast<const float*>(gr.data), gd,
-                                      static_cast<float*>(nd.out.data), p);
+                                      static_cast<float*>(nd.out.data), p, false);
         }
         case VKHIP_OP_CONV2D_INPUT_GRAD: {
             vkhip_unfold p;
@@ -758,7 +759,8 @@ static int compute_node(const vkhip_node& nd) {
                 return fail(VKHIP_ERR_UNSUPPORTED, "conv2d input grad: extents too large");
             return conv2d_input_grad(static_cast<const float*>(nd.src[0].data), to_operand(nd.src[0]),
                                      static_cast<const float*>(nd.src[1].data), nd.src[1].nb[0],
-                                     static_cast<uint32_t>(nd.out.ne[1]), static_cast<float*>(nd.out.data), p);
+                                     static_cast<uint32_t>(nd.out.ne[1]), static_cast<float*>(nd.out.data), p,
+                                     false);
         }
         case VKHIP_OP_CONV2D_WEIGHT_GRAD_SUM: {
             vkhip_unfold p;
@@ -781,7 +783,7 @@ static int compute_node(const vkhip_node& nd) {
             gd.nb[3] = 1;
             return conv2d_weight_grad_sum(static_cast<const float*>(nd.src[0].data), to_operand(nd.src[0]),
                                           static_cast<const float*>(gr.data), gd,
-                                          static_cast<float*>(nd.out.data), p);
+                                          static_cast<float*>(nd.out.data), p, false);
         }
         case VKHIP_OP_MAX_POOL2D_BACKWARD_RELU_BIAS: {
             const vkhip_tensor& y = nd.src[1];

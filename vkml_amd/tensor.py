@@ -150,14 +150,15 @@ class DeviceBackend:
 
     def transposed_plans_agree(self, batch: int, m: int, n: int, k: int) -> bool:
         """Whether the M x N and N x M products over the same K get the same
-        bits for the same products: the same split-K plan (the library's fp32
-        kernels sum each output's K range in an order only the plan decides)
-        on kernels that treat both operands alike
-        (vkhip_gemm_transposable)."""
+        split-K plan, and so the same bits for the same products (a node's
+        product runs on the library's fp32 kernels, which sum each output's K
+        range in an order only the plan's (splits, chunk) decides)."""
         key = (batch, m, n, k)
         hit = self._plans.get(key)
         if hit is None:
-            hit = bool(self.hip.lib.vkhip_gemm_transposable(batch, m, n, k))
+            from . import ops
+
+            hit = ops.gemm_plan(batch, m, n, k) == ops.gemm_plan(batch, n, m, k)
             self._plans[key] = hit
         return hit
 
