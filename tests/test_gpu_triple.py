@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from conftest import SEED, gemm_tolerance, normwise_rel_err
-from vkml_amd import ops
+from vkml_amd import _lib, ops
 from vkml_amd import tensor as T
 from vkml_amd.device import DeviceArray, DecisionRecorder
 
@@ -149,3 +149,17 @@ def test_graph_nodes_keep_the_fp32_kernels(hip):
     ones = np.ones((1000, 1501))
     for grad, exact in ((got[4], ones @ v), (got[5], ones.T @ u)):
         assert normwise_rel_err(grad, exact) <= gemm_tolerance(1501)
+
+
+def test_a_forced_kernel_or_split_stays_on_the_fp32_cores(hip):
+    rng = np.random.default_rng(SEED + 5)
+    a, b = (_view(rng.standard_normal(s).astype(np.float32), "n") for s in ((1000, 777), (777, 1501)))
+    with DecisionRecorder() as rec:
+        auto = ops.matmul(a, b).numpy()
+    assert _operand_kinds(rec) == ["three_bf16_terms"]
+    with DecisionRecorder() as rec:
+        forced = ops.matmul(a, b, kernel=_lib.GEMM_MFMA).numpy()
+        unsplit = ops.matmul(a, b, split_k=1).numpy()
+    assert _operand_kinds(rec) == []
+    assert ops.gemm_plan(1, 1000, 1501, 777)[0] == 1 and np.array_equal(forced, unsplit)
+    assert not np.array_equal(forced, auto)

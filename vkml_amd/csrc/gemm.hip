@@ -2655,7 +2655,7 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
                   : (g.sbn == 1 && aligned(b, g.sb0, g.sb1, g.sbk));
 
     const uint64_t out_elems = batch * m * n;
-    if (terms && split_req == 0) {
+    if (terms && kernel == VKHIP_GEMM_AUTO && split_req == 0) {
         const TriplePlan t = triple_plan(static_cast<uint32_t>(batch), m, n, k);
         if (t) {
             publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, t.chunk, t.slices);
