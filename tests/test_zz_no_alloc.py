@@ -75,3 +75,19 @@ def test_noalloc_gemm_refuses_a_split_beyond_its_scratch(hip):
     assert code == _lib.OK
     code, want = _gemm("vkhip_gemm", a, b, 0)
     assert got.tobytes() == want.tobytes()
+
+
+def test_a_requested_split_folded_in_one_launch_needs_no_scratch(hip):
+    """64x40000x512 as four requested partitions: 41 MB of partials if they
+    were written, but one wave per partition folds them in the workgroup."""
+    from vkml_amd import ops
+
+    assert ops.gemm_plan(1, 64, 40000, 512, 4) == (4, 4)
+    assert 4 * 64 * 40000 * 4 > 32 << 20
+    a, b = _operands(64, 40000, 512, 11)
+    code, got = _gemm("vkhip_gemm_noalloc", a, b, 4)
+    assert code == _lib.OK, _lib.load().vkhip_last_error()
+    parts = [ops.matmul(DeviceArray((64, 128), a.dtype, a.strides, a.buffer, 128 * p),
+                        DeviceArray((128, 40000), b.dtype, b.strides, b.buffer, 128 * p * 40000), split_k=1).numpy()
+             for p in range(4)]
+    assert np.array_equal(got, (parts[0] + parts[1]) + (parts[2] + parts[3]))

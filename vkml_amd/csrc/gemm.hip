@@ -2706,7 +2706,8 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
     // for a single pair); every other kernel one per partition.
     const bool direct128 = tile.bm == 128 && b_rows && (amode == KCD || a_rows);
     const bool paired = direct128 && tile.pair && splits >= 2 && reinterpret_cast<uintptr_t>(c) % 16 == 0;
-    if (split_req == 0 && small_fits(static_cast<uint32_t>(batch), m, n, splits, chunk, tile)) {
+    if ((split_req == 0 || (splits > 1 && tile.bm == 64)) &&
+        small_fits(static_cast<uint32_t>(batch), m, n, splits, chunk, tile)) {
         g.tiles_m = ceil_div(m, 32u);
         g.tiles_n = ceil_div(n, 32u);
         g.c = c;
