@@ -163,3 +163,19 @@ def test_a_forced_kernel_or_split_stays_on_the_fp32_cores(hip):
     assert _operand_kinds(rec) == []
     assert ops.gemm_plan(1, 1000, 1501, 777)[0] == 1 and np.array_equal(forced, unsplit)
     assert not np.array_equal(forced, auto)
+
+
+def test_sums_of_one_term_are_rounded_as_in_fp32(hip):
+    """A diagonal matrix times a matrix is one product per output. The operands'
+    lower terms are as large as they get (1 + 2^-8 - 2^-17 and its neighbours),
+    so every term product but l * l' (2^-34 of the product) shows: half an ulp,
+    2^-24, plus that and its few roundings."""
+    n = 2048
+    d = np.full(n, 0x3f807fc0, np.int32).view(np.float32)
+    b = (0x3f807fc0 + np.arange(-n // 2, n // 2, dtype=np.int32)).view(np.float32)
+    b = np.broadcast_to(b, (n, n)).copy()
+    with DecisionRecorder() as rec:
+        got = ops.matmul(_view(np.diag(d), "n"), _view(b, "n")).numpy()
+    assert _operand_kinds(rec) == ["three_bf16_terms"]
+    exact = d.astype(np.float64)[:, None] * b.astype(np.float64)
+    assert np.max(np.abs(got - exact) / exact) <= 2.0 ** -24 * (1 + 2.0 ** -7)

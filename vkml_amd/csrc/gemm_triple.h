@@ -1,16 +1,17 @@
 // fp32 products on the bf16 matrix cores. An fp32 value x is exactly the sum
 // of three bf16 terms, x = h + m + l: h the nearest bf16 to x, m the nearest to
 // x - h, l = x - h - m (24 significant bits, at least 8 per term). The product
-// of two such sums has nine term products; six are computed (hl', lh', mm',
-// hm', mh', hh', each exact in fp32) and summed in fp32 by
-// v_mfma_f32_32x32x16_bf16. The three left out (ml', lm', ll') are at most
-// 2^-26 of the product, below the 2^-24 rounding of one fp32 addition. A K
-// step of 16 takes six MFMAs of 32 cycles against eight of 64 for
-// v_mfma_f32_32x32x2_f32, and rounds an accumulator six times against eight.
+// of two such sums has nine term products; all but ll' are computed, each exact
+// in fp32, and summed in fp32 by v_mfma_f32_32x32x16_bf16. |m| reaches 2^-8 of
+// x and |l| 2^-17, so ll' is at most 2^-34 of the product, while ml' and lm'
+// together reach 2^-24: without them a sum of one non-zero term (a diagonal
+// matrix, a selection) was off by up to 1.2e-7 of it, twice fp32's rounding;
+// with them by 5.97e-8. A K step of 16 takes eight MFMAs of 32 cycles against
+// eight of 64 for v_mfma_f32_32x32x2_f32.
 //
 // The matrix core drops the bits of a product that lie too far below the
 // accumulator it is added to, always downwards: added to the sum of the hh'
-// products, the five smaller ones left it too small by a mean of 0.06 to 0.2 of
+// products, the smaller ones left it too small by a mean of 0.06 to 0.2 of
 // its (random) error, which shows where many outputs are summed again (2.3e-6
 // of a bias gradient, 6e-7 on the fp32 cores). They have an accumulator of
 // their own: the mean is below 0.02 of the error (a bias gradient 1.2e-7), and
@@ -441,8 +442,8 @@ struct TripleTile {
     // it can run beside them.
     template <class F>
     __device__ __forceinline__ void multiply(Lds cur, F&& next) {
-        // smallest products first: hl' lh' mm' hm' mh' hh'
-        constexpr int TA[6] = {0, 2, 1, 0, 1, 0}, TB[6] = {2, 0, 1, 1, 0, 0};
+        // smallest products first: ml' lm' hl' lh' mm' hm' mh' hh'
+        constexpr int TA[8] = {1, 2, 0, 2, 1, 0, 1, 0}, TB[8] = {2, 1, 2, 0, 1, 1, 0, 0};
         bf16x8 fa[3][MI], fb[3][NI];
 #pragma unroll
         for (int p = 0; p < 3; ++p)
@@ -454,12 +455,12 @@ struct TripleTile {
             for (int i = 0; i < MI; ++i) fa[p][i] = ra.read(cur, p, i);
         next();
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
+        for (int q = 0; q < 8; ++q)
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int j = 0; j < NI; ++j) {
-                    f32x16& c = q < 5 ? cor[i][j] : acc[i][j];
+                    f32x16& c = q < 7 ? cor[i][j] : acc[i][j];
                     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[TA[q]][i], fb[TB[q]][j], c, 0, 0, 0);
                 }
     }
