@@ -179,3 +179,19 @@ def test_sums_of_one_term_are_rounded_as_in_fp32(hip):
     assert _operand_kinds(rec) == ["three_bf16_terms"]
     exact = d.astype(np.float64)[:, None] * b.astype(np.float64)
     assert np.max(np.abs(got - exact) / exact) <= 2.0 ** -24 * (1 + 2.0 ** -7)
+
+
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 16384), (130, 780, 16400)])
+def test_split_plans_keep_their_partitions(hip, m, n, k):
+    """A product whose K the plan splits is summed partition by partition: long
+    chains of products of one sign lose more than the fp32 kernels do."""
+    assert ops.gemm_plan(1, m, n, k)[0] > 2
+    rng = np.random.default_rng(SEED + 7)
+    a, b = (np.maximum(rng.standard_normal(s), 0).astype(np.float32) for s in ((m, k), (k, n)))
+    with DecisionRecorder() as rec:
+        got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    assert _operand_kinds(rec) == []
+    rows = np.arange(0, m, 16)
+    fp32 = ops.matmul(_view(a, "n"), _view(b, "n"), kernel=_lib.GEMM_MFMA).numpy()[rows]
+    exact = a[rows].astype(np.float64) @ b.astype(np.float64)
+    assert normwise_rel_err(got[rows], exact) <= normwise_rel_err(fp32, exact)

@@ -2280,12 +2280,9 @@ int gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k, int32_t split_
 }
 
 // ---- products on the bf16 matrix cores (gemm_triple.h) --------------------------
-// Whether an AUTO product runs there, on which square tile, and how many
-// consecutive partitions of its split-K plan each workgroup takes as one chain
-// (`run`; run * chunk K-tiles, slices = ceil(splits / run) partials).
+// The tile of an AUTO product that runs there.
 struct TriplePlan {
     int tile = -1;  // kTripleTiles; negative: the fp32 matrix cores
-    uint32_t slices = 1, chunk = 1;
     explicit operator bool() const { return tile >= 0; }
 };
 
@@ -2303,13 +2300,11 @@ static const TripleTileTimes kTripleTiles[] = {{64, 64, 0.20, 0.285, 0.225, "64x
                                                {128, 128, 0.55, 0.75, 0.69, "128x128 tiles"},
                                                {256, 128, 0.90, 1.27, 1.27, "256x128 tiles"}};
 
-// Microseconds of a launch of `tiles` x `slices` workgroups of `stages` stages.
-static double triple_time(const TripleTileTimes& t, uint64_t tiles, uint32_t slices, uint32_t stages,
-                          uint64_t out_elems, double cus) {
-    const double w = static_cast<double>(tiles) * slices / cus;
+// Microseconds of a launch of `tiles` workgroups of `stages` stages.
+static double triple_time(const TripleTileTimes& t, uint64_t tiles, uint32_t stages, double cus) {
+    const double w = static_cast<double>(tiles) / cus;
     const double per = w <= 1.0 ? t.one + (t.full - t.one) * w : t.share * std::ceil(w);
-    const double fold = slices > 1 ? 4.5 + 8.0 * slices * static_cast<double>(out_elems) / 5e6 : 0.0;
-    return 4.0 + stages * per + fold;
+    return 4.0 + stages * per;
 }
 
 // Products of more than this many multiply-adds take them. Below, the launch
@@ -2327,6 +2322,14 @@ constexpr double kTripleMinMacs = 268435456.0;
 // nor for batches of tall shallow products, the columns of a strided input
 // gradient, all output: [20,96,32,32] -> 96 3x3 stride 2 (20 of 864x256x96)
 // 38.9 and 45.1, [64,64,32,32] -> 128 (64 of 576x256x128) 67.3 and 73.8.
+//
+// Nor for a product whose K the fp32 plan splits. Its partitions are short
+// chains, added up at the end: as long chains the three terms were less exact
+// where every product is of one sign (relu(N) against relu(N), 1024x1024x16384
+// 1.64e-7 of the result, fp32 1.30e-7), and as short ones no faster
+// (1024x1024x4096 94 us, fp32 84; 256x256x65536 97 and 85; 128x784x16384 49 and
+// 44). Two partitions of 64x64 tiles are the exception, since the two groups of
+// stages of the 64x64 tile are two such chains: 1024^3 25.4 us, fp32 33.7.
 static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
     TriplePlan best;
     if (m <= 32 || n <= 32 || k < 64) return best;
@@ -2335,47 +2338,33 @@ static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k
     uint32_t splits, chunk;
     TileChoice plan;
     gemm_plan(batch, m, n, k, 0, splits, chunk, plan, true);
-    // no more partials than the fp32 kernels of the same plan write: pairs of
-    // partitions there leave one, and two partitions of 64x64 tiles none
-    const uint32_t most = plan.pair ? (splits + 1) / 2 : splits == 2 && plan.bm == 64 ? 1u : splits;
+    if (splits > 2 || (splits == 2 && plan.bm != 64)) return best;
     const double cus = ctx().ready ? ctx().caps.compute_units : 256.0;
-    const uint64_t out_elems = static_cast<uint64_t>(batch) * m * n;
-    const uint32_t ktotal = ceil_div(k, 16u);
     double best_us = 1e30;
-    for (int tile = 0; tile < 3; ++tile) {
+    uint64_t wgs = 0;
+    for (int tile = 0; tile < (splits == 1 ? 3 : 1); ++tile) {
         const TripleTileTimes& tt = kTripleTiles[tile];
         const uint64_t tiles = static_cast<uint64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch;
-        // slice counts about 1.4 apart: 1, 2, 3, 4, 6, 8, 12, ...
-        for (uint32_t want = 1; want <= most; want = want == 1 ? 2 : (want & (want - 1)) == 0 ? want * 3 / 2 : want / 3 * 4) {
-            const uint32_t run = (splits + want - 1) / want;
-            const uint32_t slices = (splits + run - 1) / run;
-            const uint32_t stages = std::min(ktotal, 2 * run * chunk);
-            const double us = triple_time(tt, tiles, slices, stages, out_elems, cus);
-            if (us < best_us) {
-                best_us = us;
-                best.tile = tile;
-                best.slices = slices;
-                best.chunk = run * chunk;
-            }
+        const double us = triple_time(tt, tiles, ceil_div(k, 16u), cus);
+        if (us < best_us) {
+            best_us = us;
+            best.tile = tile;
+            wgs = tiles;
         }
     }
-    const TripleTileTimes& tt = kTripleTiles[best.tile];
-    const uint64_t wgs = static_cast<uint64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch * best.slices;
     if (2.0 * wgs <= cus || (std::min(m, n) <= 64 && k <= 320) || (batch > 1 && m > 128 && k <= 128)) return TriplePlan{};
     return best;
 }
 
-// Launches a product planned there; g holds the operands, strides and sizes,
-// and when the plan has one slice the epilogue. `c` is the output of one slice
-// or the partials of several.
+// Launches a product planned there; g holds the operands, strides, sizes and
+// output.
 static int launch_triple_product(GemmArgs& g, const Im2colB& im, const TriplePlan& t, uint32_t batch, int am, int bm) {
     g.tiles_m = ceil_div(g.m, kTripleTiles[t.tile].bm);
     g.tiles_n = ceil_div(g.n, kTripleTiles[t.tile].bn);
-    g.chunk = t.chunk;
-    const uint64_t flat = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * t.slices;
-    if (flat > 0x7fffffffull) return fail(VKHIP_ERR_UNSUPPORTED, "gemm: %llu workgroups", static_cast<unsigned long long>(flat));
-    g.flat_splits = t.slices > 1 ? t.slices : 0;
-    const dim3 grid(static_cast<uint32_t>(flat), 1, batch);
+    g.flat_splits = 0;
+    const uint64_t tiles = static_cast<uint64_t>(g.tiles_m) * g.tiles_n;
+    if (tiles > 0x7fffffffull) return fail(VKHIP_ERR_UNSUPPORTED, "gemm: %llu workgroups", static_cast<unsigned long long>(tiles));
+    const dim3 grid(static_cast<uint32_t>(tiles), 1, batch);
     return t.tile == 0   ? launch_triple_64x64(g, im, grid, am, bm)
            : t.tile == 1 ? launch_triple_128x128(g, im, grid, am, bm)
                          : launch_triple_256x128(g, im, grid, am, bm);
@@ -2658,22 +2647,13 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
     if (terms && kernel == VKHIP_GEMM_AUTO && split_req == 0) {
         const TriplePlan t = triple_plan(static_cast<uint32_t>(batch), m, n, k);
         if (t) {
-            publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, t.chunk, t.slices);
-            float* target = c;
-            if (t.slices > 1) {
-                const int st = partials(out_elems * t.slices * sizeof(float), &target);
-                if (st != VKHIP_OK) return st;
-                g.split_stride = out_elems;
-            } else {
-                g.epi = fe;
-            }
+            publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, m, n);
             *fused = true;
-            g.c = target;
+            g.epi = fe;
+            g.c = c;
             int am = triple_mode(m, k, g.sam, g.sak), bm = triple_mode(n, k, g.sbn, g.sbk);
             if (am == TG || bm == TG) am = bm = TG;
-            const int st = launch_triple_product(g, Im2colB{}, t, static_cast<uint32_t>(batch), am, bm);
-            if (st != VKHIP_OK || t.slices == 1) return st;
-            return launch_split_k_reduce(target, c, out_elems, t.slices, fe);
+            return launch_triple_product(g, Im2colB{}, t, static_cast<uint32_t>(batch), am, bm);
         }
     }
     int amode = akc ? (g.a_vec ? KCV : KCS) : (g.a_vec ? RCV : RCS);
@@ -3608,7 +3588,7 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     // the plan gemm() takes for the same product, so the same bits
     const TriplePlan triple = terms && triple_mode(m, k, g.sam, g.sak) == TK
                                   ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
-    if (triple) splits = triple.slices;
+    if (triple) splits = 1;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -3640,7 +3620,7 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     const uint64_t w64 = static_cast<uint64_t>(g.tiles_m) * ceil_div(n, 64) * splits * batch;
     if (triple) {
         publish("matmul.operands", "conv2d", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
-                triple.chunk, triple.slices);
+                m, n);
         st = launch_triple_product(g, im, triple, static_cast<uint32_t>(batch), TK, TI);
     } else if (tile.bm == 128 && 0.94 * round_fill(w64, 2 * cus) > round_fill(w128, 2 * cus)) {
         g.tiles_n = ceil_div(n, 64);
@@ -3778,7 +3758,7 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     float* target = out;
     const TriplePlan triple = terms && g.sa1 >= 0 && triple_mode(m, k, g.sam, g.sak) == TK && triple_image_fits(im, oh)
                                   ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
-    if (triple) splits = triple.slices;
+    if (triple) splits = 1;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -3790,7 +3770,7 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     int st;
     if (triple) {
         publish("matmul.operands", "conv2d_weight_grad", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
-                triple.chunk, triple.slices);
+                m, n);
         st = launch_triple_product(g, im, triple, static_cast<uint32_t>(batch), TK, TT);
     } else if (tile.bm == 128 && wgrad_direct_fits(g, k, target)) {
         // both operands straight into LDS (same bits as the register path);
@@ -4050,19 +4030,6 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     const int amode = g.a_vec ? KCV : KCS;
     const uint64_t out_elems = static_cast<uint64_t>(m) * n;
     float* target = out;
-    // Where 32-deep K-tiles stay inside an image the fp32 kernels are ahead of
-    // the three terms, which gather and split the columns once per row of tiles
-    // ([48,64,16,16] -> 128 3x3 44.9 us against 49.1, [32,64,32,32] -> 64 55.2
-    // and 61.3, [24,96,16,16] -> 96 37.0 and 40.9); where they cross images
-    // behind ([64,32,28,28] -> 64 3x3 54.2 and 37.1, [32,128,14,14] -> 96 41.1
-    // and 36.4), and where two rows of tiles share a gather over a deep K
-    // (K 32768, [128,64,16,16] -> 128 3x3 63.6 and 55.3, and 65536, [64,128,32,32] -> 128 1x1
-    // 42.5 and 33.6; K 12288 is the 44.9 against 49.1 above).
-    const TriplePlan triple = terms && (L % 32 != 0 || (std::min(m, n) > 64 && k >= 32768)) && g.sa1 >= 0 &&
-                                      triple_mode(m, static_cast<uint32_t>(L), g.sam, g.sak) == TK &&
-                                      triple_image_fits(im, oh)
-                                  ? triple_plan(1, m, n, k) : TriplePlan{};
-    if (triple) splits = triple.slices;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -4072,11 +4039,7 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     g.c = target;
     g.split_stride = splits > 1 ? out_elems : 0;
     int st;
-    if (triple) {
-        publish("matmul.operands", "conv2d_weight_grad_sum", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
-                triple.chunk, triple.slices);
-        st = launch_triple_product(g, im, triple, 1, TKB, TTB);
-    } else if (tile.bm == 128 && wgrad_direct_fits(g, static_cast<uint32_t>(L), target)) {
+    if (tile.bm == 128 && wgrad_direct_fits(g, static_cast<uint32_t>(L), target)) {
         const bool narrow = wgrad_narrow_tiles(g, splits, 1);
         if (narrow) g.tiles_n = ceil_div(n, 64u);
         const uint64_t flat = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * splits;
