@@ -14,7 +14,7 @@ import pytest
 
 import oracle as O
 from conftest import ROOT
-from vkml_amd import _lib
+from vkml_amd import _lib, ops
 
 HEADER = ROOT / "include" / "vkhip.h"
 
@@ -443,3 +443,25 @@ def test_program_output_order_hoists_the_output_cone_within_hazards():
     # An output nothing writes is final before the first unit.
     order, after = _output_order([fwd, bwd1], [(OTHER, 4)])
     assert order == [0, 1] and after == 0
+
+
+# (batch, m, n, k) and whether the three-term products were the faster ones where
+# both were measured (us on the fp32 kernels, with three terms)
+@pytest.mark.parametrize("shape,terms", [
+    ((1, 2100, 2300, 100), False),   # 18.7 21.4
+    ((16, 576, 256, 256), False),    # 18.3 20.3
+    ((20, 864, 256, 96), False),     # 15.7 20.6
+    ((1, 1024, 1024, 4096), False),  # 84 94, K split
+    ((4, 496, 139, 1152), False),    # 20.8 23.1, fewer tiles than CUs
+    ((32, 288, 560, 123), True),     # 35.2 23.5
+    ((16, 1872, 448, 118), True),    # 61.1 41.4
+    ((16, 272, 1232, 80), True),     # 23.0 15.8
+    ((1, 3808, 960, 6145), True),    # 758 345
+    ((1, 4096, 4096, 4096), True),   # 927 784
+])
+def test_three_term_products_lie_where_they_are_faster(shape, terms):
+    """A product whose orientations agree (vkhip_gemm_transposable) is on the
+    fp32 kernels in both; three-term products never do."""
+    batch, m, n, k = shape
+    assert ops.gemm_plan(batch, m, n, k) == ops.gemm_plan(batch, n, m, k)
+    assert bool(_lib.load().vkhip_gemm_transposable(batch, m, n, k)) is not terms

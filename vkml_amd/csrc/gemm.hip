@@ -2286,73 +2286,77 @@ struct TriplePlan {
     explicit operator bool() const { return tile >= 0; }
 };
 
-// The tiles, and microseconds per 16-deep stage of one workgroup, measured: a
-// launch of few workgroups takes `one`, a workgroup on every CU `full`, several
-// on each `share` apiece. (Per unit of work the 256x128 tile is the fastest and
-// the 64x64 tile the slowest, 4096^3 645, 690 and 915 us, so size is traded for
-// CUs left idle: 2048^3 125, 96 and 125 us, 1024^3 64, 43 and 20 us.)
-struct TripleTileTimes {
+// A launch's microseconds: `start`, then rounds of workgroups over the CUs, each
+// `step` per 16 (three terms) or 32 (fp32) k and `round` beside; `whole` of the
+// last round counts in full, and the output is written at 1 / `out` elements
+// per us. Fitted to products of 1e8 to 7e10 multiply-adds (the time within 10%
+// for nine in ten of the three-term tiles' and of the fp32 64x64 tiles', 18%
+// for the fp32 128x128 tiles'); per unit of work the 256x128 tile is the
+// fastest and the 64x64 tile the slowest, as fast as the fp32 kernels' 64x64.
+struct TileTime {
     uint32_t bm, bn;
-    double one, full, share;
+    double start, step, round, whole, out;
     const char* name;
+    double us(uint64_t tiles, uint32_t steps, double out_elems, double cus) const {
+        const double w = static_cast<double>(tiles) / cus;
+        const double rounds = w <= 1.0 ? 1.0 : whole * std::ceil(w) + (1.0 - whole) * w;
+        return start + rounds * (steps * step + round) + out * out_elems;
+    }
 };
-static const TripleTileTimes kTripleTiles[] = {{64, 64, 0.20, 0.285, 0.225, "64x64 tiles"},
-                                               {128, 128, 0.55, 0.75, 0.69, "128x128 tiles"},
-                                               {256, 128, 0.90, 1.27, 1.27, "256x128 tiles"}};
+static const TileTime kTripleTiles[] = {{64, 64, 4.9, 0.27, 1.5, 0.64, 2.4e-7, "64x64 tiles"},
+                                        {128, 128, 5.1, 0.81, 0.8, 0.68, 5.2e-7, "128x128 tiles"},
+                                        {256, 128, 2.0, 1.265, 7.0, 1.0, 7.6e-7, "256x128 tiles"}};
+static const TileTime kFp32Tiles[] = {{64, 64, 4.9, 0.53, 0.0, 0.92, 6.2e-7, ""},
+                                      {128, 128, 3.9, 1.85, 0.0, 0.48, 9.2e-7, ""}};
 
-// Microseconds of a launch of `tiles` workgroups of `stages` stages.
-static double triple_time(const TripleTileTimes& t, uint64_t tiles, uint32_t stages, double cus) {
-    const double w = static_cast<double>(tiles) / cus;
-    const double per = w <= 1.0 ? t.one + (t.full - t.one) * w : t.share * std::ceil(w);
-    return 4.0 + stages * per;
-}
+// Products of fewer multiply-adds keep the fp32 cores: the launch and the first
+// loads are most of the time on either path (128x8192x256, 2.7e8, 9.3 us there
+// and 9.8 here; 660^3, 2.9e8, 16.5 and 16.3).
+constexpr double kTripleMinMacs = 3e8;
 
-// Products of more than this many multiply-adds take them. Below, the launch
-// and the first loads are most of the time on either path: 128x8192x256 (2^28)
-// 10.7 us on the fp32 cores and 11.0 here, 1000x1000x64 11.1 and 11.0, 512^3
-// 11.4 and 12.6; above, 700^3 17.1 and 16.4, 1024^3 24.7 and 20.7.
-constexpr double kTripleMinMacs = 268435456.0;
-
-// Not for a launch that leaves half of the CUs idle (a batch, whose images are
-// not split): a convolution's workgroups there wait for their own gathers,
-// [32,96,16,16] -> 64 3x3 22.8 us on the fp32 cores and 25.5 here, [16,128,16,16]
-// -> 128 25.9 and 30.7, its columns as a product 24.4 and 22.3. Nor for one row
-// of tiles over a short K, whose epilogue weighs as much: [64,32,28,28] -> 64
-// 3x3 27.1 and 28.7 ([32,64,16,16] -> 128 3x3, twice the K, 21.0 and 18.9);
-// nor for batches of tall shallow products, the columns of a strided input
-// gradient, all output: [20,96,32,32] -> 96 3x3 stride 2 (20 of 864x256x96)
-// 38.9 and 45.1, [64,64,32,32] -> 128 (64 of 576x256x128) 67.3 and 73.8.
+// A product takes the three terms where their time is below the fp32 kernels'
+// by the model, by 8%, or within 10% of it for sizes that are not multiples of
+// four, whose fp32 loads are 4 bytes wide (3808x960x6145 758 us on the fp32
+// cores and 345 here; 1558x1712x439 91 and 56). Of 585 products and lowered
+// convolutions measured this takes 342, which run at 0.74 of their fp32 time;
+// eight of them are slower, by 3 to 11%.
+//
+// Not for fewer 64x64 tiles than CUs (a batch, whose images are not split): a
+// workgroup there waits for its own loads, [16,64,20,20] -> 128 5x5 input
+// gradient 59 us on the fp32 cores and 79 here, 4 of 496x139x1152 21 and 23.
 //
 // Nor for a product whose K the fp32 plan splits. Its partitions are short
 // chains, added up at the end: as long chains the three terms were less exact
 // where every product is of one sign (relu(N) against relu(N), 1024x1024x16384
 // 1.64e-7 of the result, fp32 1.30e-7), and as short ones no faster
 // (1024x1024x4096 94 us, fp32 84; 256x256x65536 97 and 85; 128x784x16384 49 and
-// 44). Two partitions of 64x64 tiles are the exception, since the two groups of
-// stages of the 64x64 tile are two such chains: 1024^3 25.4 us, fp32 33.7.
+// 44). Two partitions of one round of 64x64 tiles are the exception, since the
+// two groups of stages of the 64x64 tile are two such chains: 1024^3 25.4 us,
+// fp32 33.7 with B transposed and 24.7 without.
 static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
     TriplePlan best;
     if (m <= 32 || n <= 32 || k < 64) return best;
-    const double macs = static_cast<double>(batch) * m * n * k;
-    if (macs <= kTripleMinMacs) return best;
+    if (static_cast<double>(batch) * m * n * k < kTripleMinMacs) return best;
     uint32_t splits, chunk;
     TileChoice plan;
     gemm_plan(batch, m, n, k, 0, splits, chunk, plan, true);
     if (splits > 2 || (splits == 2 && plan.bm != 64)) return best;
     const double cus = ctx().ready ? ctx().caps.compute_units : 256.0;
-    double best_us = 1e30;
-    uint64_t wgs = 0;
+    const double out_elems = static_cast<double>(batch) * m * n;
+    const TileTime& fp32 = kFp32Tiles[plan.bm == 128];
+    const bool ragged = m % 4 != 0 || n % 4 != 0 || k % 4 != 0;
+    double below = (ragged ? 1.1 : 0.92) * fp32.us(plan.tiles, ceil_div(k, 32u), out_elems, cus);
+    if (splits == 2) below = 1e30;
     for (int tile = 0; tile < (splits == 1 ? 3 : 1); ++tile) {
-        const TripleTileTimes& tt = kTripleTiles[tile];
+        const TileTime& tt = kTripleTiles[tile];
         const uint64_t tiles = static_cast<uint64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch;
-        const double us = triple_time(tt, tiles, ceil_div(k, 16u), cus);
-        if (us < best_us) {
-            best_us = us;
+        if (tile == 0 && static_cast<double>(tiles) < cus) continue;
+        const double us = tt.us(tiles, ceil_div(k, 16u), out_elems, cus);
+        if (us < below) {
+            below = us;
             best.tile = tile;
-            wgs = tiles;
         }
     }
-    if (2.0 * wgs <= cus || (std::min(m, n) <= 64 && k <= 320) || (batch > 1 && m > 128 && k <= 128)) return TriplePlan{};
     return best;
 }
 
