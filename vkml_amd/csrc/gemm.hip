@@ -2652,9 +2652,7 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
         const TriplePlan t = triple_plan(static_cast<uint32_t>(batch), m, n, k);
         if (t) {
             publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, m, n);
-            *fused = true;
-            g.epi = fe;
-            g.c = c;
+            g.c = c;  // (an epilogue follows as a pass of its own)
             int am = triple_mode(m, k, g.sam, g.sak), bm = triple_mode(n, k, g.sbn, g.sbk);
             if (am == TG || bm == TG) am = bm = TG;
             return launch_triple_product(g, Im2colB{}, t, static_cast<uint32_t>(batch), am, bm);
@@ -3590,7 +3588,7 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     const uint64_t out_elems = batch * m * n;
     float* target = out;
     // the plan gemm() takes for the same product, so the same bits
-    const TriplePlan triple = terms && triple_mode(m, k, g.sam, g.sak) == TK
+    const TriplePlan triple = terms && !bias && !relu && triple_mode(m, k, g.sam, g.sak) == TK
                                   ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
     if (triple) splits = 1;
     if (splits > 1) {

@@ -604,42 +604,6 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
         for (int j = 0; j < NI; ++j) {
             uint32_t col;
             const bool col_in = OB::real_row(col0 + wn0 + 32 * j + lrow, g.n, col);
-            // Every epilogue load before the first store, and none behind a
-            // branch of its own (rows past the operand read the last row's):
-            // one memory round trip instead of sixteen (15 us less in a
-            // training step whose largest forward is 128x256x576, batch 128).
-            float out[16], with[16];
-            if constexpr (BMODE == TI) {
-                if (g.bias) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        with[r] = g.bias[static_cast<int64_t>(min(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4),
-                                                                  g.m - 1u)) * g.bias_stride];
-                }
-            }
-            if (g.epi.mask) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    uint32_t row;
-                    OA::real_row(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4), g.m, row);
-                    with[r] = g.epi.mask[(static_cast<uint64_t>(z) * g.m + min(row, g.m - 1u)) * g.n + min(col, g.n - 1u)];
-                }
-            }
-            const float col_bias =
-                g.epi.bias ? g.epi.bias[static_cast<int64_t>(min(col, g.n - 1u)) * g.epi.bias_stride] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                out[r] = acc[i][j][r];
-                if constexpr (BMODE == TI) {
-                    if (g.bias) out[r] += with[r];
-                    if (g.relu) out[r] = out[r] <= 0.0f ? 0.0f : out[r];
-                }
-                if (g.epi.bias) {
-                    out[r] += col_bias;
-                    if (g.epi.relu) out[r] = out[r] <= 0.0f ? 0.0f : out[r];
-                }
-                if (g.epi.mask && with[r] <= 0.0f) out[r] = 0.0f;
-            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 uint32_t row;
@@ -648,9 +612,9 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
                     // outputs of large tiles and convolutions are read by
                     // later kernels only
                     if constexpr (BM >= 128 || BMODE >= TI)
-                        __builtin_nontemporal_store(out[r], at);
+                        __builtin_nontemporal_store(acc[i][j][r], at);
                     else
-                        *at = out[r];
+                        *at = acc[i][j][r];
                 }
             }
         }
