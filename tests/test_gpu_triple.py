@@ -195,3 +195,25 @@ def test_split_plans_keep_their_partitions(hip, m, n, k):
     fp32 = ops.matmul(_view(a, "n"), _view(b, "n"), kernel=_lib.GEMM_MFMA).numpy()[rows]
     exact = a[rows].astype(np.float64) @ b.astype(np.float64)
     assert normwise_rel_err(got[rows], exact) <= normwise_rel_err(fp32, exact)
+
+
+def test_tiny_inputs_among_ordinary_ones_change_nothing(hip):
+    """Inputs below 2^-110 lose low bits as terms, nothing beside outputs of
+    ordinary size: those keep the bits they have with zeros in their place. An
+    output made of such inputs alone has fp32's accuracy."""
+    rng = np.random.default_rng(SEED + 9)
+    m, n, k = 1000, 1501, 777
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    a[:, 5] = 0.0
+    want = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    a[::7, 5] = 1e-36
+    b[3, ::11] *= np.float32(1e-38)
+    zeroed = b.copy()
+    zeroed[3, ::11] = 0.0
+    want[:, ::11] = ops.matmul(_view(a, "n"), _view(zeroed, "n")).numpy()[:, ::11]
+    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    assert np.count_nonzero(got.view(np.uint32) != want.view(np.uint32)) == 0
+    a[130] = rng.standard_normal(k) * 1e-35
+    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    exact = a[130].astype(np.float64) @ b.astype(np.float64)
+    assert normwise_rel_err(got[130], exact) <= 8e-7

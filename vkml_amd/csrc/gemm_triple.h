@@ -18,10 +18,16 @@
 // the sum of the hh' products is rounded once per 16 k.
 //
 // What the terms cannot hold is computed again in fp32. Inf and NaN inputs, and
-// values that round up to inf as h, make every output they reach non-finite;
-// an input with 0 < |x| < 2^-110 may have l below bf16's smallest value 2^-133.
-// A workgroup that ends with a non-finite accumulator, or has staged such an
-// input, runs its K range again on v_mfma_f32_32x32x2_f32 and keeps that.
+// values that round up to inf as h, make every output they reach non-finite: a
+// workgroup that ends with a non-finite accumulator runs its K range again on
+// v_mfma_f32_32x32x2_f32 and keeps that. The terms of an input with 0 < |x| <
+// 2^-110 may end at bf16's smallest value 2^-133 and so leave out up to 2^-134
+// of it. All such inputs together change an output by at most K 2^-133 of the
+// largest input, so a workgroup that has staged one reads its operands again for
+// that and runs again only where an output is below K 2^-103 of it, 2^30 times
+// as much. (4096^3 on one box: 0.87 ms; with such an input in every tile, a
+// probability of 1e-34 among ordinary ones, 1.12, and 2.36 with a second pass
+// for all of them; 0.93 on the fp32 matrix cores.)
 //
 // Error of N(0,1) products against 64 bits (relative, 2-norm), the fp32 matrix
 // cores' in brackets: 1024^3 1.9e-7 (4.1e-7, K in two partitions), 2048^3
@@ -384,6 +390,18 @@ struct TripleStager {
         a.put(stage, va[d], tiny);
         b.put(stage + OA::kBytes, vb[d], tiny);
     }
+    __device__ __forceinline__ uint32_t largest(int d) const {
+        uint32_t most = 0;
+#pragma unroll
+        for (int i = 0; i < OA::NG; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) most = max(most, __builtin_bit_cast(uint32_t, va[d][i][j]) & 0x7fffffffu);
+#pragma unroll
+        for (int i = 0; i < OB::NG; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) most = max(most, __builtin_bit_cast(uint32_t, vb[d][i][j]) & 0x7fffffffu);
+        return most;
+    }
     __device__ __forceinline__ void put32(Lds stage, int d) const {
         a.put32(stage, va[d], t);
         b.put32(stage + OA::kBytes32, vb[d], t);
@@ -481,6 +499,21 @@ struct TripleTile {
         }
     }
 
+    // The bits of the largest magnitude this thread's loads have had.
+    template <class S>
+    __device__ __forceinline__ uint32_t largest(S& st, const Im2colB& im) {
+        uint32_t most = 0;
+#pragma unroll 1
+        for (int s = 0; s < ns + (tail ? 1 : 0); ++s) {
+            if (s == ns)
+                st.template fetch<true>(0, full, im);
+            else
+                st.template fetch<false>(0, stage_of(s), im);
+            most = max(most, st.largest(0));
+        }
+        return most;
+    }
+
     // The same stages and order of groups in fp32.
     template <class S>
     __device__ __forceinline__ void run32(S& st, Lds lds, const Im2colB& im, int wm0, int wn0, int lane) {
@@ -556,21 +589,35 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
 
     tile.gather();
     auto& acc = tile.acc;
+    // (rows past an operand's end hold whatever the LDS held)
+    auto inside = [&](int i, int j, int r) {
+        uint32_t row, col;
+        return OA::real_row(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4), g.m, row) &&
+               OB::real_row(col0 + wn0 + 32 * j + lrow, g.n, col);
+    };
     float finite = 0.0f;  // becomes NaN with any non-finite accumulator of the output
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                // (rows past an operand's end hold whatever the LDS held)
-                uint32_t row, col;
-                const bool inside = OA::real_row(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4), g.m, row) &&
-                                    OB::real_row(col0 + wn0 + 32 * j + lrow, g.n, col);
-                finite = __builtin_fmaf(inside ? acc[i][j][r] : 0.0f, 0.0f, finite);
-            }
-    if (__syncthreads_or(!(finite == 0.0f) || tiny < kTripleTiny))
-        tile.run32(st, lds, im, wm0, wn0, lane);
+            for (int r = 0; r < 16; ++r) finite = __builtin_fmaf(inside(i, j, r) ? acc[i][j][r] : 0.0f, 0.0f, finite);
+    if (__syncthreads_or(!(finite == 0.0f) || tiny < kTripleTiny)) {
+        uint32_t* most = reinterpret_cast<uint32_t*>(lds_all);
+        if (threadIdx.x == 0) *most = 0u;
+        __syncthreads();
+        atomicMax(most, tile.largest(st, im));
+        __syncthreads();
+        const float bound = static_cast<float>(g.k) * 0x1p-103f * __builtin_bit_cast(float, *most);
+        bool far = finite == 0.0f;  // every output far above what the tiny inputs lose
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) far = far && (!inside(i, j, r) || __builtin_fabsf(acc[i][j][r]) >= bound);
+        if (__syncthreads_or(!far)) tile.run32(st, lds, im, wm0, wn0, lane);
+    }
     if constexpr (KG > 1) {
         float* part = reinterpret_cast<float*>(lds_all);
         __syncthreads();
