@@ -259,8 +259,11 @@ typedef struct vkhip_copy {
 /* ---- GEMM selection knobs: the reference's VKML_GEMM_* switches
  *      (vulkan_backend.cpp:536-561, 2160-2250) as explicit arguments ------- */
 enum vkhip_gemm_kernel {
-    VKHIP_GEMM_AUTO = 0,   /* MFMA tiles, split-K / GEMV by the planner */
-    VKHIP_GEMM_MFMA = 1,   /* MFMA tiles, never GEMV */
+    /* MFMA tiles, split-K / GEMV by the planner; large products of vkhip_gemm,
+     * vkhip_gemm_noalloc and the conv entry points as sums of three bf16 terms
+     * per operand, no less exact than the fp32 matrix cores (nodes: never) */
+    VKHIP_GEMM_AUTO = 0,
+    VKHIP_GEMM_MFMA = 1,   /* fp32 MFMA tiles, never GEMV or terms */
     VKHIP_GEMM_GEMV = 2,   /* force the GEMV path (N == 1 or M == 1 only) */
     /* the comparison arm: each product rounded, the K products summed in the
      * CPU oracle's pairwise order, so C is the oracle's bit for bit (the role
@@ -353,7 +356,7 @@ int vkhip_compute(const vkhip_node* nodes, size_t n);
 /* ======================================================================== */
 
 /* C[b0,b1,M,N] (contiguous) = A[b0,b1,M,K] @ B[b0,b1,K,N]; any strides
- * (NN / NT / TN / batch-broadcast). fp32 in, fp32 MFMA accumulate.
+ * (NN / NT / TN / batch-broadcast). fp32 in, fp32 accumulate in the MFMA.
  * Reference: Matmul case, vulkan_backend.cpp:2056-2657; CPU oracle
  * kernels_matmul.cpp:34-87. `opts` may be NULL (AUTO). */
 int vkhip_gemm(const float* a, const vkhip_operand* a_desc,
@@ -380,8 +383,8 @@ int vkhip_gemm_noalloc(const float* a, const vkhip_operand* a_desc,
  * no split) and chunk (K-tiles per partition, a power of two). */
 int vkhip_gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k,
                     int32_t split_request, uint32_t* out_splits, uint32_t* out_chunk);
-/* 1 when AUTO gives the M x N product A @ B and the N x M product B^T @ A^T
- * over the same K the same bits (equal plans, and a kernel whose sums do not
+/* 1 when AUTO gives vkhip_gemm's M x N product A @ B and the N x M product
+ * B^T @ A^T over the same K the same bits (equal plans, and a kernel whose sums do not
  * depend on which operand comes first), else 0. Callable without a GPU. */
 int vkhip_gemm_transposable(uint32_t batch, uint32_t m, uint32_t n, uint32_t k);
 
@@ -517,7 +520,9 @@ int vkhip_sgd_step(const vkhip_sgd_param* params, size_t count, float lr, float 
 /* ======================================================================== */
 /* One choice the backend made, what it rejected, why, and the numbers that
  * forced it (reference vkml::observe::Decision, include/vkml/util/observe.h:
- * 55-93). Sites: "matmul.kernel", "matmul.split_k", "reduce.structure",
+ * 55-93). Sites: "matmul.kernel", "matmul.split_k" (products on the fp32
+ * matrix cores), "matmul.operands" (products as three bf16 terms; their kernels
+ * are gemm_triple_<tile>, unsplit), "conv.input_grad", "reduce.structure",
  * "softmax.structure", "col2im.kernel", "max_pool2d.kernel",
  * "allocator.release". The strings live for the duration of the callback
  * only. `dispatch` names the unit of work the choice produced: the same id the

@@ -217,3 +217,16 @@ def test_tiny_inputs_among_ordinary_ones_change_nothing(hip):
     got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
     exact = a[130].astype(np.float64) @ b.astype(np.float64)
     assert normwise_rel_err(got[130], exact) <= 8e-7
+
+
+def test_decisions_name_the_kernel_that_runs(hip):
+    a, b = DeviceArray((1000, 777)), DeviceArray((777, 1501))
+    with DecisionRecorder() as rec:
+        ops.matmul(a, b)
+    by_site = {d["site"]: d for d in rec.decisions}
+    kernel = by_site["matmul.kernel"]
+    assert (kernel["chose"], kernel["instead_of"]) == ("gemm_triple_64x64", "gemm_mfma_64x64")
+    assert (kernel["required"], kernel["available"]) == (16 * 24, hip.capabilities().compute_units)
+    operands = by_site["matmul.operands"]
+    assert (operands["required"], operands["available"], operands["dispatch"]) == (1000, 1501, kernel["dispatch"])
+    assert "matmul.split_k" not in by_site

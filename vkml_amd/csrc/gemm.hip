@@ -2303,9 +2303,9 @@ struct TileTime {
         return start + rounds * (steps * step + round) + out * out_elems;
     }
 };
-static const TileTime kTripleTiles[] = {{64, 64, 4.9, 0.27, 1.5, 0.64, 2.4e-7, "64x64 tiles"},
-                                        {128, 128, 5.1, 0.81, 0.8, 0.68, 5.2e-7, "128x128 tiles"},
-                                        {256, 128, 2.0, 1.265, 7.0, 1.0, 7.6e-7, "256x128 tiles"}};
+static const TileTime kTripleTiles[] = {{64, 64, 4.9, 0.27, 1.5, 0.64, 2.4e-7, "gemm_triple_64x64"},
+                                        {128, 128, 5.1, 0.81, 0.8, 0.68, 5.2e-7, "gemm_triple_128x128"},
+                                        {256, 128, 2.0, 1.265, 7.0, 1.0, 7.6e-7, "gemm_triple_256x128"}};
 static const TileTime kFp32Tiles[] = {{64, 64, 4.9, 0.53, 0.0, 0.92, 6.2e-7, ""},
                                       {128, 128, 3.9, 1.85, 0.0, 0.48, 9.2e-7, ""}};
 
@@ -2358,6 +2358,16 @@ static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k
         }
     }
     return best;
+}
+
+// The decision of such a product: its kernel, the fp32 one it stands for, its
+// tiles and the CUs they fill, and its operands.
+static void publish_triple(const char* op, const TriplePlan& t, const char* instead, uint32_t batch, uint32_t m, uint32_t n) {
+    const TileTime& tt = kTripleTiles[t.tile];
+    const char* because = "the three-term time is below the fp32 kernels'";
+    publish("matmul.kernel", op, tt.name, instead, because,
+            static_cast<int64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch, ctx().ready ? ctx().caps.compute_units : 256);
+    publish("matmul.operands", op, "three_bf16_terms", "fp32", because, m, n);
 }
 
 // Launches a product planned there; g holds the operands, strides, sizes and
@@ -2600,7 +2610,12 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
         *ws = scratch->ptr;
         return VKHIP_OK;
     };
-    {
+    const TriplePlan triple = terms && kernel == VKHIP_GEMM_AUTO && split_req == 0
+                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
+    if (triple) {
+        publish_triple("matmul", triple, tile.bm == 128 ? "gemm_mfma_128x128" : "gemm_mfma_64x64",
+                       static_cast<uint32_t>(batch), m, n);
+    } else {
         const int64_t cus = ctx().ready ? ctx().caps.compute_units : 256;
         publish("matmul.kernel", "matmul", tile.bm == 128 ? "gemm_mfma_128x128" : "gemm_mfma_64x64",
                 tile.bm == 128 ? "gemm_mfma_64x64" : "gemm_mfma_128x128", tile.why,
@@ -2648,15 +2663,11 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
                   : (g.sbn == 1 && aligned(b, g.sb0, g.sb1, g.sbk));
 
     const uint64_t out_elems = batch * m * n;
-    if (terms && kernel == VKHIP_GEMM_AUTO && split_req == 0) {
-        const TriplePlan t = triple_plan(static_cast<uint32_t>(batch), m, n, k);
-        if (t) {
-            publish("matmul.operands", "matmul", "three_bf16_terms", "fp32", kTripleTiles[t.tile].name, m, n);
-            g.c = c;  // (an epilogue follows as a pass of its own)
-            int am = triple_mode(m, k, g.sam, g.sak), bm = triple_mode(n, k, g.sbn, g.sbk);
-            if (am == TG || bm == TG) am = bm = TG;
-            return launch_triple_product(g, Im2colB{}, t, static_cast<uint32_t>(batch), am, bm);
-        }
+    if (triple) {
+        g.c = c;  // (an epilogue follows as a pass of its own)
+        int am = triple_mode(m, k, g.sam, g.sak), bm = triple_mode(n, k, g.sbn, g.sbk);
+        if (am == TG || bm == TG) am = bm = TG;
+        return launch_triple_product(g, Im2colB{}, triple, static_cast<uint32_t>(batch), am, bm);
     }
     int amode = akc ? (g.a_vec ? KCV : KCS) : (g.a_vec ? RCV : RCS);
     // The buffer-load paths (straight-to-LDS operands and the direct kernels)
@@ -3548,10 +3559,18 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     uint32_t splits, chunk;
     TileChoice tile;
     gemm_plan(static_cast<uint32_t>(batch), m, n, k, 0, splits, chunk, tile);
-    publish("matmul.kernel", "conv2d", tile.bm == 128 ? "gemm_mfma_128x128_implicit_im2col"
-                                                      : "gemm_mfma_64x64_implicit_im2col",
-            "im2col_then_gemm", "the cols matrix is gathered from the image inside the GEMM",
-            static_cast<int64_t>(tile.tiles), ctx().ready ? ctx().caps.compute_units : 256);
+    const bool weight_rows = triple_mode(m, k, wd.nb[2], 1) == TK;
+    // the plan gemm() takes for the same product, so the same bits
+    const TriplePlan triple = terms && !bias && !relu && weight_rows
+                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
+    const char* const fp32_kernel = tile.bm == 128 ? "gemm_mfma_128x128_implicit_im2col"
+                                                   : "gemm_mfma_64x64_implicit_im2col";
+    if (triple)
+        publish_triple("conv2d", triple, fp32_kernel, static_cast<uint32_t>(batch), m, n);
+    else
+        publish("matmul.kernel", "conv2d", fp32_kernel, "im2col_then_gemm",
+                "the cols matrix is gathered from the image inside the GEMM",
+                static_cast<int64_t>(tile.tiles), ctx().ready ? ctx().caps.compute_units : 256);
 
     GemmArgs g{};
     g.a = w;
@@ -3587,9 +3606,6 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
 
     const uint64_t out_elems = batch * m * n;
     float* target = out;
-    // the plan gemm() takes for the same product, so the same bits
-    const TriplePlan triple = terms && !bias && !relu && triple_mode(m, k, g.sam, g.sak) == TK
-                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
     if (triple) splits = 1;
     if (splits > 1) {
         float* ws = nullptr;
@@ -3621,8 +3637,6 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     const uint64_t w128 = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * splits * batch;
     const uint64_t w64 = static_cast<uint64_t>(g.tiles_m) * ceil_div(n, 64) * splits * batch;
     if (triple) {
-        publish("matmul.operands", "conv2d", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
-                m, n);
         st = launch_triple_product(g, im, triple, static_cast<uint32_t>(batch), TK, TI);
     } else if (tile.bm == 128 && 0.94 * round_fill(w64, 2 * cus) > round_fill(w128, 2 * cus)) {
         g.tiles_n = ceil_div(n, 64);
@@ -3726,10 +3740,16 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     uint32_t splits, chunk;
     TileChoice tile;
     gemm_plan(static_cast<uint32_t>(batch), m, n, k, 0, splits, chunk, tile);
-    publish("matmul.kernel", "conv2d_weight_grad",
-            tile.bm == 128 ? "gemm_mfma_128x128_implicit_im2col_t" : "gemm_mfma_64x64_implicit_im2col_t",
-            "im2col_then_gemm", "the transposed cols matrix is gathered from the image inside the GEMM",
-            static_cast<int64_t>(tile.tiles), ctx().ready ? ctx().caps.compute_units : 256);
+    const TriplePlan triple = terms && gd.nb[1] >= 0 && triple_mode(m, k, gd.nb[2], 1) == TK && triple_image_fits(im, oh)
+                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
+    const char* const fp32_kernel = tile.bm == 128 ? "gemm_mfma_128x128_implicit_im2col_t"
+                                                   : "gemm_mfma_64x64_implicit_im2col_t";
+    if (triple)
+        publish_triple("conv2d_weight_grad", triple, fp32_kernel, static_cast<uint32_t>(batch), m, n);
+    else
+        publish("matmul.kernel", "conv2d_weight_grad", fp32_kernel, "im2col_then_gemm",
+                "the transposed cols matrix is gathered from the image inside the GEMM",
+                static_cast<int64_t>(tile.tiles), ctx().ready ? ctx().caps.compute_units : 256);
     im.x = x;
     im.sn = xd.nb[0];
 
@@ -3758,8 +3778,6 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     const int amode = a_kcd ? KCD : (g.a_vec ? KCV : KCS);
     const uint64_t out_elems = batch * m * n;
     float* target = out;
-    const TriplePlan triple = terms && g.sa1 >= 0 && triple_mode(m, k, g.sam, g.sak) == TK && triple_image_fits(im, oh)
-                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
     if (triple) splits = 1;
     if (splits > 1) {
         float* ws = nullptr;
@@ -3771,8 +3789,6 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     g.split_stride = splits > 1 ? out_elems : 0;
     int st;
     if (triple) {
-        publish("matmul.operands", "conv2d_weight_grad", "three_bf16_terms", "fp32", kTripleTiles[triple.tile].name,
-                m, n);
         st = launch_triple_product(g, im, triple, static_cast<uint32_t>(batch), TK, TT);
     } else if (tile.bm == 128 && wgrad_direct_fits(g, k, target)) {
         // both operands straight into LDS (same bits as the register path);
