@@ -1,5 +1,6 @@
 """Products on the bf16 matrix cores (gemm_triple.h): three-term operands, all
-layouts the same bits, and the fp32 pass for what the terms cannot hold."""
+layouts the same bits, and the fp32 pass for what the terms cannot hold. Every
+test asserts which kernel its products took."""
 from __future__ import annotations
 
 import numpy as np
@@ -31,49 +32,95 @@ def _view(x: np.ndarray, how: str) -> DeviceArray:
     return DeviceArray.from_numpy(x)
 
 
-# (batch, m, n, k): 64, 128 and 256 tiles; one row or column past a tile, less
-# than four rows in the last tile, a last stage of 1, 9 and 15 k, split K
-SHAPES = [(1, 1000, 1501, 777), (1, 257, 2049, 1025), (1, 4099, 3841, 89), (3, 515, 641, 319),
-          (1, 67, 130, 40001), (1, 33, 4100, 2100), (16, 129, 131, 1040)]
+def _operand_kinds(rec: DecisionRecorder) -> list[str]:
+    return [d["chose"] for d in rec.decisions if d["site"] == "matmul.operands"]
 
 
-@pytest.mark.parametrize("batch,m,n,k", SHAPES)
-def test_layouts_and_edges(hip, batch, m, n, k):
+def _three_terms(a: DeviceArray, b: DeviceArray, kernel: str | None = None) -> np.ndarray:
+    """a @ b, which must run as three-term products (on the given kernel)."""
+    with DecisionRecorder() as rec:
+        out = ops.matmul(a, b).numpy()
+    assert _operand_kinds(rec) == ["three_bf16_terms"]
+    took = [d["chose"] for d in rec.decisions if d["site"] == "matmul.kernel"]
+    assert took == [kernel] if kernel else took[0].startswith("gemm_triple_")
+    return out
+
+
+def _off(got: np.ndarray, exact: np.ndarray) -> float:
+    """The relative error in the 2-norm."""
+    return float(np.linalg.norm(got - exact) / np.linalg.norm(exact))
+
+
+def _bound(k: int) -> float:
+    """_off of N(0,1) products: each 16 k round the sum once,
+    by at most 2^-24 of a partial sum, whose mean square is half of the last one's
+    or less; the roundings are independent. Plus half an ulp of the result. (For
+    every k here below 8e-7; a product without its third terms is off by 2.4e-6.)"""
+    return 2.0 ** -24 * (1 + 0.5 * np.sqrt(k / 16))
+
+
+# (kernel, batch, m, n, k): one or three rows or columns past a tile, fewer than
+# four rows in the last tile, a last stage of 1, 9 and 15 k, and none
+SHAPES = [("64x64", 1, 1000, 1501, 777), ("64x64", 3, 515, 641, 319), ("64x64", 1, 1025, 1089, 1040),
+          ("128x128", 1, 4099, 3841, 89), ("128x128", 16, 257, 389, 417), ("128x128", 1, 2051, 3842, 100),
+          ("256x128", 16, 257, 897, 257), ("256x128", 16, 1535, 130, 321), ("256x128", 16, 1795, 130, 223)]
+
+
+@pytest.mark.parametrize("tile,batch,m,n,k", SHAPES)
+def test_layouts_and_edges(hip, tile, batch, m, n, k):
     rng = np.random.default_rng(SEED + m + n + k)
     lead = (batch,) if batch > 1 else ()
     a = rng.standard_normal(lead + (m, k), dtype=np.float32)
     b = rng.standard_normal(lead + (k, n), dtype=np.float32)
     print(f"triple {batch} {m}x{n}x{k}", flush=True)
-    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    got = _three_terms(_view(a, "n"), _view(b, "n"), f"gemm_triple_{tile}")
     rows = np.unique(np.r_[0:4, m // 2, m - 4:m])
     exact = a[..., rows, :].astype(np.float64) @ b.astype(np.float64)
-    assert normwise_rel_err(got[..., rows, :], exact) <= min(gemm_tolerance(k), 2.0 ** -23 * np.sqrt(k))
+    assert _off(got[..., rows, :], exact) <= _bound(k)
     for la, lb in (("n", "t"), ("t", "n"), ("t", "t"), ("o", "o"), ("r", "n"), ("n", "r")):
-        same = ops.matmul(_view(a, la), _view(b, lb)).numpy()
+        same = _three_terms(_view(a, la), _view(b, lb), f"gemm_triple_{tile}")
         differ = int(np.count_nonzero(same.view(np.uint32) != got.view(np.uint32)))
         assert differ == 0, (la, lb)
 
 
-@pytest.mark.parametrize("m,n,k", [(1000, 700, 600), (2100, 2300, 100)])
+@pytest.mark.parametrize("m,n,k", [(1000, 1501, 777), (4099, 3841, 89)])
 @pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1e36), (1e30, 1e-30), (3e-39, 1.0), (1e-20, 1e-19)])
 def test_scales_keep_fp32_accuracy(hip, m, n, k, scale_a, scale_b):
-    """Operands of any fp32 scale, subnormals included: the fp32 product's
-    accuracy (relative, or one part in 2^24 of the smallest normal number)."""
+    """Operands of any fp32 scale, subnormals included: the accuracy of the
+    terms, or where they cannot hold the operands of the fp32 pass, whose sum is
+    rounded every two k (and one part in 2^24 of the smallest normal number)."""
     rng = np.random.default_rng(SEED + m)
     a = (rng.standard_normal((m, k)) * scale_a).astype(np.float32)
     b = (rng.standard_normal((k, n)) * scale_b).astype(np.float32)
     print(f"triple scale {scale_a} {scale_b}", flush=True)
-    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy().astype(np.float64)
-    exact = a.astype(np.float64) @ b.astype(np.float64)
-    off = np.linalg.norm(got - exact)
-    assert off <= 2.0 ** -23 * np.sqrt(k) * np.linalg.norm(exact) + 2.0 ** -149 * k * np.sqrt(m * n)
+    got = _three_terms(_view(a, "n"), _view(b, "n"))[::8].astype(np.float64)
+    exact = a[::8].astype(np.float64) @ b.astype(np.float64)
+    terms = min(scale_a, scale_b) > 1e-22  # no input below 2^-110
+    assert np.linalg.norm(got - exact) <= (_bound(k if terms else 8 * k) * np.linalg.norm(exact)
+                                           + 2.0 ** -149 * k * np.sqrt(exact.size))
+
+
+def test_lower_terms_below_the_smallest_normal_number(hip):
+    """Inputs of 2^-108: their third terms are subnormal bf16 values, which the
+    conversion and the matrix cores have to keep (3e-6 of the result if not)."""
+    rng = np.random.default_rng(SEED + 1)
+    m, n, k = 1000, 1501, 777
+
+    def signed(shape, scale):
+        return (rng.uniform(1, 2, shape) * rng.choice([-1, 1], shape) * scale).astype(np.float32)
+
+    a, b = signed((m, k), 2.0 ** -109), signed((k, n), 2.0 ** 100)
+    for x, y in ((a, b), (np.ascontiguousarray(b.T), np.ascontiguousarray(a.T))):
+        got = _three_terms(_view(x, "n"), _view(y, "n"))[::8]
+        exact = x[::8].astype(np.float64) @ y.astype(np.float64)
+        assert _off(got, exact) <= _bound(k)
 
 
 def test_infinities_nans_and_the_largest_values(hip):
     """Where a 64-bit product is finite in fp32, the result is it; elsewhere
     infinities and NaNs land where IEEE arithmetic puts them."""
     rng = np.random.default_rng(SEED)
-    m, n, k = 600, 640, 800
+    m, n, k = 1100, 1300, 801
     a = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
     b = rng.uniform(0.5, 1.5, (k, n)).astype(np.float32)
     a[3, 5] = np.inf
@@ -84,7 +131,7 @@ def test_infinities_nans_and_the_largest_values(hip):
     b[7, 300] = 0.5
     b[20, 64] = np.inf
     a[200, 20] = 0.0                      # 0 * inf
-    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    got = _three_terms(_view(a, "n"), _view(b, "n"))
     with np.errstate(invalid="ignore", over="ignore"):
         exact = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
     np.testing.assert_array_equal(np.isnan(got), np.isnan(exact))
@@ -94,8 +141,10 @@ def test_infinities_nans_and_the_largest_values(hip):
     np.testing.assert_allclose(got[fine], exact[fine], rtol=1e-5)
 
 
-@pytest.mark.parametrize("n,c,hw,cout,window,stride", [(37, 40, (19, 23), 70, 3, 1), (9, 65, (30, 31), 130, 5, 2),
-                                                      (64, 33, (32, 32), 257, 3, 1)])
+# forward on the 128x128, 64x64 and 256x128 tiles, weight gradient on 64x64,
+# 256x128 and 128x128
+@pytest.mark.parametrize("n,c,hw,cout,window,stride", [(64, 33, (32, 32), 257, 3, 1), (33, 33, (30, 31), 130, 5, 2),
+                                                       (64, 40, (14, 14), 258, 3, 1)])
 def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stride):
     rng = np.random.default_rng(SEED + c)
     x = rng.uniform(-1, 1, (n, c) + hw).astype(np.float32)
@@ -105,22 +154,22 @@ def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stri
     print(f"triple conv {x.shape} {cout}", flush=True)
     cols = ops.im2col(dx, window, stride, pad)
     _, ck, L = cols.shape
-    got = ops.conv2d(dx, dw, stride, pad)
-    want = ops.matmul(dw.reshape(1, 1, cout, ck).broadcast_to((1, n, cout, ck)), cols.reshape(1, n, ck, L))
+    with DecisionRecorder() as rec:
+        got = ops.conv2d(dx, dw, stride, pad)
+        want = ops.matmul(dw.reshape(1, 1, cout, ck).broadcast_to((1, n, cout, ck)), cols.reshape(1, n, ck, L))
+    assert _operand_kinds(rec) == ["three_bf16_terms"] * 2
     assert np.array_equal(got.numpy().reshape(-1), want.numpy().reshape(-1))
     g = rng.standard_normal(got.shape).astype(np.float32)
     dg = DeviceArray.from_numpy(g)
-    per = ops.conv2d_weight_grad(dx, dg, window, stride, pad)
-    want = ops.matmul(dg.reshape(1, n, cout, L), cols.reshape(1, n, ck, L).transpose(-2, -1)).numpy()
+    with DecisionRecorder() as rec:
+        per = ops.conv2d_weight_grad(dx, dg, window, stride, pad)
+        want = ops.matmul(dg.reshape(1, n, cout, L), cols.reshape(1, n, ck, L).transpose(-2, -1)).numpy()
+    assert _operand_kinds(rec) == ["three_bf16_terms"] * 2
     assert np.array_equal(per.numpy().reshape(-1), want.reshape(-1))
     total = ops.conv2d_weight_grad_sum(dx, dg, window, stride, pad).numpy()
     exact = np.einsum("nol,nkl->ok", g.reshape(n, cout, L).astype(np.float64), cols.numpy().astype(np.float64),
                       optimize=True)
     assert normwise_rel_err(total, exact) <= 2.0 ** -23 * np.sqrt(n * L)
-
-
-def _operand_kinds(rec: DecisionRecorder) -> list[str]:
-    return [d["chose"] for d in rec.decisions if d["site"] == "matmul.operands"]
 
 
 def test_graph_nodes_keep_the_fp32_kernels(hip):
@@ -154,9 +203,7 @@ def test_graph_nodes_keep_the_fp32_kernels(hip):
 def test_a_forced_kernel_or_split_stays_on_the_fp32_cores(hip):
     rng = np.random.default_rng(SEED + 5)
     a, b = (_view(rng.standard_normal(s).astype(np.float32), "n") for s in ((1000, 777), (777, 1501)))
-    with DecisionRecorder() as rec:
-        auto = ops.matmul(a, b).numpy()
-    assert _operand_kinds(rec) == ["three_bf16_terms"]
+    auto = _three_terms(a, b)
     with DecisionRecorder() as rec:
         forced = ops.matmul(a, b, kernel=_lib.GEMM_MFMA).numpy()
         unsplit = ops.matmul(a, b, split_k=1).numpy()
@@ -174,9 +221,7 @@ def test_sums_of_one_term_are_rounded_as_in_fp32(hip):
     d = np.full(n, 0x3f807fc0, np.int32).view(np.float32)
     b = (0x3f807fc0 + np.arange(-n // 2, n // 2, dtype=np.int32)).view(np.float32)
     b = np.broadcast_to(b, (n, n)).copy()
-    with DecisionRecorder() as rec:
-        got = ops.matmul(_view(np.diag(d), "n"), _view(b, "n")).numpy()
-    assert _operand_kinds(rec) == ["three_bf16_terms"]
+    got = _three_terms(_view(np.diag(d), "n"), _view(b, "n"))
     exact = d.astype(np.float64)[:, None] * b.astype(np.float64)
     assert np.max(np.abs(got - exact) / exact) <= 2.0 ** -24 * (1 + 2.0 ** -7)
 
@@ -194,7 +239,7 @@ def test_split_plans_keep_their_partitions(hip, m, n, k):
     rows = np.arange(0, m, 16)
     fp32 = ops.matmul(_view(a, "n"), _view(b, "n"), kernel=_lib.GEMM_MFMA).numpy()[rows]
     exact = a[rows].astype(np.float64) @ b.astype(np.float64)
-    assert normwise_rel_err(got[rows], exact) <= normwise_rel_err(fp32, exact)
+    assert _off(got[rows], exact) <= _off(fp32, exact)
 
 
 def test_tiny_inputs_among_ordinary_ones_change_nothing(hip):
@@ -205,18 +250,18 @@ def test_tiny_inputs_among_ordinary_ones_change_nothing(hip):
     m, n, k = 1000, 1501, 777
     a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
     a[:, 5] = 0.0
-    want = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    want = _three_terms(_view(a, "n"), _view(b, "n"))
     a[::7, 5] = 1e-36
     b[3, ::11] *= np.float32(1e-38)
     zeroed = b.copy()
     zeroed[3, ::11] = 0.0
-    want[:, ::11] = ops.matmul(_view(a, "n"), _view(zeroed, "n")).numpy()[:, ::11]
-    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    want[:, ::11] = _three_terms(_view(a, "n"), _view(zeroed, "n"))[:, ::11]
+    got = _three_terms(_view(a, "n"), _view(b, "n"))
     assert np.count_nonzero(got.view(np.uint32) != want.view(np.uint32)) == 0
     a[130] = rng.standard_normal(k) * 1e-35
-    got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    got = _three_terms(_view(a, "n"), _view(b, "n"))
     exact = a[130].astype(np.float64) @ b.astype(np.float64)
-    assert normwise_rel_err(got[130], exact) <= 8e-7
+    assert _off(got[130], exact) <= _bound(8 * k)  # the fp32 pass rounds every two k
 
 
 def test_decisions_name_the_kernel_that_runs(hip):
