@@ -30,8 +30,10 @@
 // for all of them; 0.93 on the fp32 matrix cores.)
 //
 // Error of N(0,1) products against 64 bits (relative, 2-norm), the fp32 matrix
-// cores' in brackets: 1024^3 1.9e-7 (4.1e-7, K in two partitions), 2048^3
-// 2.7e-7 (8.1e-7), 4096^3 4.0e-7 (1.1e-6).
+// cores' in brackets: 1024^3 1.3e-7 (4.1e-7), 2048^3 2.7e-7 (8.1e-7), 4096^3
+// 4.0e-7 (1.15e-6). Operands of one sign, uniform in 0..1: 0.9e-7 (2.2e-7),
+// 2.2e-7 (6.0e-7), 3.0e-7 (8.4e-7), with a mean of -4e-9 of the sum at 4096^3
+// (-4e-9) from the floors; relu(N) on both sides 3.2e-7 (4.9e-7) at 4096^3.
 //
 // Layout: a stage is 16 k of a tile's rows of both operands, three planes (h,
 // m, l) of 32 bytes per row in LDS, double buffered; the loads run D stages
@@ -46,13 +48,14 @@
 // their accumulators added in LDS in order.
 //
 // What bounds it: power, then the splitting and the LDS reads per MFMA. A loop
-// of nothing but these MFMAs reaches 1.45-1.7 PFLOP/s of bf16 on this card
-// (the clock falls to about 1.7 GHz), 240-280 TFLOP/s of fp32 products; the
-// 256x128 tile runs 4096^3 at 213 (645 us; 930 on the fp32 cores). Counted with
-// one accumulator, the matrix cores were busy 72% of the cycles with 128x128
-// tiles at 4096^3 and 54% at one workgroup per CU (2048^3, 96 us; 126): a
-// stage of the 128x128 tile reads 72 KB and writes 24 KB of LDS for 768 cycles
-// of MFMAs, of the 64x64 tile half of that for a quarter of the MFMAs.
+// of nothing but these MFMAs reaches 1.45-1.7 PFLOP/s of bf16 on this card, 180
+// to 210 TFLOP/s of fp32 products; the 256x128 tile runs 4096^3 at 170 (810 us;
+// 930 on the fp32 cores). Counted there, the matrix cores are busy 69% of the
+// cycles, at a clock of 1.73 GHz; at 2048^3 (128x128 tiles, one workgroup per
+// CU, 120 us; 126) 50%, at 1024^3 22%: a stage of the 128x128 tile reads 72 KB
+// and writes 24 KB of LDS for 1024 cycles of MFMAs, of the 64x64 tile half of
+// that for a quarter of the MFMAs. The 128x128 tile's 128 registers, for two
+// workgroups per CU, spill up to seven values around the loop, none inside it.
 #pragma once
 
 #include <algorithm>
