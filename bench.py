@@ -6,7 +6,8 @@ one GEMM. Prints ONE JSON line:
 
   value        whole-job TFLOP/s over the timed K steps (2*M*N*K per step)
   roofline     the GEMM kernel's algorithmic TFLOP/s from HIP-event launch times
-               on the backend's stream, against the bf16 MFMA peak over six (416.7 TFLOP/s)
+               on the backend's stream, against the peak of the matrix cores it runs on
+               (fp32: 157.3 TFLOP/s; three bf16 terms: the bf16 peak over eight, 312.5)
   cpu_baseline the CPU oracle (the C restatement of vkML's CPU matmul) on a row
                sample of the same problem, on this host's cores
   secondary    the other hot-path kernels at their BASELINE shapes (GB/s against
@@ -39,9 +40,9 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 MFMA_FP32_PEAK_TFLOPS = 157.3
-# The headline product runs as six bf16 term products: the dense bf16 peak
-# (2.5 PFLOP/s) over six, in fp32 multiply-adds.
-TRIPLE_PEAK_TFLOPS = 2500.0 / 6
+# Large products run as eight bf16 term products: the dense bf16 peak
+# (2.5 PFLOP/s) over eight, in fp32 multiply-adds.
+TRIPLE_PEAK_TFLOPS = 2500.0 / 8
 HBM_PEAK_GBS = 8000.0
 # fp32 VALU rate for rounded multiplies and adds issued separately (no FMA, no
 # packed fp32): 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz, one FLOP per lane-op.
@@ -110,6 +111,18 @@ def gate(launches: int = 24):
         ops.matmul(a, a, out=c)
 
 
+def matrix_roof(fn) -> tuple[float, str]:
+    """The peak (TFLOP/s) of the matrix cores that fn's product runs on, and its
+    kernel, from the library's decision facts of one call."""
+    from vkml_amd.device import DecisionRecorder
+
+    with DecisionRecorder() as rec:
+        fn()
+    triple = any(d["chose"] == "three_bf16_terms" for d in rec.decisions)
+    kernel = [d["chose"] for d in rec.decisions if d["site"] == "matmul.kernel"]
+    return TRIPLE_PEAK_TFLOPS if triple else MFMA_FP32_PEAK_TFLOPS, kernel[-1] if kernel else ""
+
+
 def time_launches(fn, timer: Timer, reps: int, warmup: int = 3):
     """Per-launch durations (ms) from event pairs around each call (for
     launches long enough that event overhead is negligible)."""
@@ -167,7 +180,8 @@ def gemm_headline(args, hip, ops, timer):
     value = flop * args.steps / wall / 1e12
     avg_ms = float(np.mean(launch_ms))
     achieved = flop / (avg_ms * 1e-3) / 1e12
-    return value, wall * 1e3 / args.steps, avg_ms, achieved, float(np.min(launch_ms)), done
+    peak, kernel = matrix_roof(lambda: ops.matmul(a, b, out=c))
+    return value, wall * 1e3 / args.steps, avg_ms, achieved, float(np.min(launch_ms)), done, peak, kernel
 
 
 def _cpu_model() -> str:
@@ -368,10 +382,11 @@ def case_gemm(name, hip, ops, timer, rng, out):
     bv = b if lay[1] == "n" else b.T
     c = DeviceArray((m, n), np.float32)
     ms = time_batch(lambda i: ops.matmul(av, bv, out=c), timer, 10 if m * n * k > 2**36 else 20)
-    splits, _ = ops.gemm_plan(1, m, n, k)
+    peak, kernel = matrix_roof(lambda: ops.matmul(av, bv, out=c))
+    splits = 1 if peak == TRIPLE_PEAK_TFLOPS else ops.gemm_plan(1, m, n, k)[0]
     tf = 2.0 * m * n * k / ms / 1e9
-    out[name] = {"ms": round(ms, 5), "tflops": round(tf, 2),
-                 "frac_of_peak": round(tf / MFMA_FP32_PEAK_TFLOPS, 4), "splits": splits}
+    out[name] = {"ms": round(ms, 5), "tflops": round(tf, 2), "kernel": kernel, "peak": peak,
+                 "frac_of_peak": round(tf / peak, 4), "splits": splits}
 
 
 def case_gemm_exact(name, hip, ops, timer, rng, out):
@@ -447,10 +462,13 @@ def case_conv(name, hip, ops, timer, rng, out):
     xs_shape, cout = CONV_CASES[name]
     n_, cin, h, w_ = xs_shape
 
-    def roof(entry, flops, byt, ms):
-        """frac_of_roofline: the larger of the two floors (MFMA FLOP, HBM
-        bytes read + written once) over the measured time; `bound` names it."""
-        t_flop = flops / (MFMA_FP32_PEAK_TFLOPS * 1e9)
+    def roof(entry, flops, byt, ms, fn):
+        """frac_of_roofline: the larger of the two floors (MFMA FLOP at the peak
+        of the matrix cores fn's product runs on, HBM bytes read + written
+        once) over the measured time; `bound` names it."""
+        entry["peak"], entry["kernel"] = matrix_roof(fn)
+        entry["frac_of_peak"] = round(flops / ms / 1e9 / entry["peak"], 4)
+        t_flop = flops / (entry["peak"] * 1e9)
         t_byte = byt / (HBM_PEAK_GBS * 1e6)
         entry["algorithmic_bytes"] = int(byt)
         entry["bound"] = "hbm" if t_byte > t_flop else "mfma"
@@ -466,7 +484,8 @@ def case_conv(name, hip, ops, timer, rng, out):
     cols = DeviceArray((n_, ck, L), np.float32)
     wf = wt.reshape(1, 1, cout, ck).broadcast_to((1, n_, cout, ck))
     flops = 2.0 * n_ * cout * L * ck
-    ms_i = time_batch(lambda i: ops.conv2d(x, wt, 1, 1, out=y), timer, 20)
+    forward = lambda i=0: ops.conv2d(x, wt, 1, 1, out=y)
+    ms_i = time_batch(forward, timer, 20)
 
     def explicit(i):
         ops.im2col(x, 3, 1, 1, out=cols)
@@ -474,14 +493,14 @@ def case_conv(name, hip, ops, timer, rng, out):
 
     ms_e = time_batch(explicit, timer, 20)
     out[name] = {"ms": round(ms_i, 5), "tflops": round(flops / ms_i / 1e9, 2),
-                 "frac_of_peak": round(flops / ms_i / 1e9 / MFMA_FP32_PEAK_TFLOPS, 4),
                  "explicit_ms": round(ms_e, 5), "speedup_vs_explicit": round(ms_e / ms_i, 3)}
-    roof(out[name], flops, x_bytes + w_bytes + y_bytes, ms_i)
+    roof(out[name], flops, x_bytes + w_bytes + y_bytes, ms_i, forward)
     g = DeviceArray.from_numpy(rng.standard_normal((n_, cout, h, w_), dtype=np.float32))
     wg = DeviceArray((n_, cout, ck), np.float32)
     g4 = g.reshape(1, n_, cout, L)
     colsT = cols.reshape(1, n_, ck, L).transpose(-2, -1)
-    ms_i = time_batch(lambda i: ops.conv2d_weight_grad(x, g, 3, 1, 1, out=wg), timer, 20)
+    per_image = lambda i=0: ops.conv2d_weight_grad(x, g, 3, 1, 1, out=wg)
+    ms_i = time_batch(per_image, timer, 20)
 
     def explicit_wg(i):
         ops.im2col(x, 3, 1, 1, out=cols)
@@ -490,10 +509,9 @@ def case_conv(name, hip, ops, timer, rng, out):
     ms_e = time_batch(explicit_wg, timer, 20)
     out[name.replace("conv_", "conv_wgrad_")] = {
         "ms": round(ms_i, 5), "tflops": round(flops / ms_i / 1e9, 2),
-        "frac_of_peak": round(flops / ms_i / 1e9 / MFMA_FP32_PEAK_TFLOPS, 4),
         "explicit_ms": round(ms_e, 5), "speedup_vs_explicit": round(ms_e / ms_i, 3)}
     roof(out[name.replace("conv_", "conv_wgrad_")], flops,
-         x_bytes + y_bytes + 4 * n_ * cout * cin * 9, ms_i)
+         x_bytes + y_bytes + 4 * n_ * cout * cin * 9, ms_i, per_image)
     # dW itself (summed over the batch): the per-image products followed by
     # the batch SUM (the reference graph's two nodes) against one product
     # with the batch folded into K
@@ -504,12 +522,12 @@ def case_conv(name, hip, ops, timer, rng, out):
         ops.sum(wg, [0], out=dw)
 
     ms_s = time_batch(per_image_then_sum, timer, 20)
-    ms_f = time_batch(lambda i: ops.conv2d_weight_grad_sum(x, g, 3, 1, 1, out=dw), timer, 20)
+    summed = lambda i=0: ops.conv2d_weight_grad_sum(x, g, 3, 1, 1, out=dw)
+    ms_f = time_batch(summed, timer, 20)
     out[name.replace("conv_", "conv_dw_")] = {
         "ms": round(ms_f, 5), "tflops": round(flops / ms_f / 1e9, 2),
-        "frac_of_peak": round(flops / ms_f / 1e9 / MFMA_FP32_PEAK_TFLOPS, 4),
         "per_image_then_sum_ms": round(ms_s, 5), "speedup_vs_per_image": round(ms_s / ms_f, 3)}
-    roof(out[name.replace("conv_", "conv_dw_")], flops, x_bytes + y_bytes + w_bytes, ms_f)
+    roof(out[name.replace("conv_", "conv_dw_")], flops, x_bytes + y_bytes + w_bytes, ms_f, summed)
     # dX: the reference graph's TN product into the column matrix and col2im,
     # against one convolution of the gradient with the flipped weight
     dx = DeviceArray(xs_shape, np.float32)
@@ -519,12 +537,12 @@ def case_conv(name, hip, ops, timer, rng, out):
         ops.col2im(cols, (h, w_), 3, 1, 1, out=dx)
 
     ms_t = time_batch(tn_then_col2im, timer, 20)
-    ms_f = time_batch(lambda i: ops.conv2d_input_grad(g, wt, (h, w_), 1, 1, out=dx), timer, 20)
+    input_grad = lambda i=0: ops.conv2d_input_grad(g, wt, (h, w_), 1, 1, out=dx)
+    ms_f = time_batch(input_grad, timer, 20)
     out[name.replace("conv_", "conv_dx_")] = {
         "ms": round(ms_f, 5), "tflops": round(flops / ms_f / 1e9, 2),
-        "frac_of_peak": round(flops / ms_f / 1e9 / MFMA_FP32_PEAK_TFLOPS, 4),
         "tn_then_col2im_ms": round(ms_t, 5), "speedup_vs_tn_col2im": round(ms_t / ms_f, 3)}
-    roof(out[name.replace("conv_", "conv_dx_")], flops, y_bytes + w_bytes + x_bytes, ms_f)
+    roof(out[name.replace("conv_", "conv_dx_")], flops, y_bytes + w_bytes + x_bytes, ms_f, input_grad)
 
 
 SOFTMAX_CASES = {"softmax_4096x1000": ((4096, 1000), 20), "softmax_256x32768": ((256, 32768), 10)}
@@ -800,17 +818,19 @@ CASES["train_mlp"] = case_training
 CASES["train_cnn"] = case_training
 
 
-def read_traffic(args):
+def read_traffic(args, kernel: str):
     """HBM bytes per launch of the headline GEMM, from the committed rocprofv3
     PMC summary (FETCH_SIZE + WRITE_SIZE, each scaled by the copy-kernel
-    calibration in the same summary); None when no summary matches."""
+    calibration in the same summary); None when no summary is of this size and
+    kernel."""
     path = ROOT / "profiles" / f"gemm_nn_{args.m}x{args.n}x{args.k}_pmc.md"
     if not path.exists():
         return None
-    for line in path.read_text().splitlines():
-        if line.startswith("traffic_bytes_per_launch:"):
-            return float(line.split(":", 1)[1])
-    return None
+    facts = dict(line.split(":", 1) for line in path.read_text().splitlines()
+                 if line.startswith(("traffic_kernel:", "traffic_bytes_per_launch:")))
+    if facts.get("traffic_kernel", "").strip() != kernel:
+        return None
+    return float(facts["traffic_bytes_per_launch"])
 
 
 def main():
@@ -831,7 +851,7 @@ def main():
         names = [c for c in args.case.split(",") if c]
         print(json.dumps({"cases": secondary(hip, ops, timer, names), "gate": _GATE_ON}), flush=True)
         return
-    value, ms_step, avg_ms, achieved, min_ms, warm = gemm_headline(args, hip, ops, timer)
+    value, ms_step, avg_ms, achieved, min_ms, warm, peak, kernel = gemm_headline(args, hip, ops, timer)
     result = {
         "metric": METRIC,
         "value": round(value, 3),
@@ -849,9 +869,9 @@ def main():
         "config": {"workload": f"gemm_nn_{args.m}x{args.n}x{args.k}_fp32", "m": args.m,
                    "n": args.n, "k": args.k, "layout": "NN", "parallelism": "none"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3),
-                     "peak": round(TRIPLE_PEAK_TFLOPS, 1), "unit": "TFLOP/s",
-                     "frac": round(achieved / TRIPLE_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": "gemm_triple_kernel",
+                     "peak": round(peak, 1), "unit": "TFLOP/s",
+                     "frac": round(achieved / peak, 4), "traffic": None,
+                     "kernel": kernel,
                      "avg_launch_ms": round(avg_ms, 4), "min_launch_ms": round(min_ms, 4)},
     }
     if args.calibrate:
@@ -861,7 +881,7 @@ def main():
         for _ in range(5):
             hip.copy_device_to_device([(dst, src)])
         hip.synchronize()
-    traffic = read_traffic(args)
+    traffic = read_traffic(args, kernel)
     if traffic is not None:
         result["roofline"]["traffic"] = traffic
     if not args.no_secondary:
