@@ -2014,13 +2014,17 @@ struct TileChoice {
 // two, or on 64x64 tiles): 4 partitions of 4 K-tiles 512^3 7.8 / 8.3 (8.6 /
 // 15.6), 333x777x211 8.7 / 8.7 (15.7 / 15.7), 8 of 2 100x1000x500 7.9 / 7.9
 // (9.0 / 8.8), 7 of 3 256x512x600 8.9 / 8.7 (9.9 / 9.9); not 13 of 2 64x128x784
-// 10.1 / 10.8 (7.1 / 6.9), 6 of 6 300x500x1000 13.8 / 13.4 (12.3 / 12.5).
+// 10.1 / 10.8 (7.1 / 6.9), 6 of 6 300x500x1000 13.8 / 13.4 (12.3 / 12.5), 8 of
+// 3 16 x 88x52x748 9.9 (9.0).
 // Unsplit: 128x784x64 4.4 / 4.2 (4.8 / 4.7), 64x10x128 5.9 / 5.3 (6.6 / 5.6);
 // not 1024x1024x128 7.2 / 7.8 (6.5 / 6.4), whose 1024 waves of 4 K-tiles do
-// better sharing their operands through LDS.
+// better sharing their operands through LDS. A ragged last K-tile costs a wave
+// 16 bounded loads per operand, so that unsplit products of a few K-tiles with
+// aligned operands are better off there too (gemm_core; NN / TN, 84x496x28 4.9
+// / 5.1, 4.3 / 4.3 there; unaligned, 42x736x35 5.1 / 5.3, 6.1 / 6.2 there).
 static bool small_fits(uint32_t batch, uint32_t m, uint32_t n, uint32_t splits, uint32_t chunk, const TileChoice& tile) {
     const uint64_t t32 = static_cast<uint64_t>(ceil_div(m, 32u)) * ceil_div(n, 32u) * batch;
-    if (splits > 1) return !tile.pair && splits <= 8 && chunk <= 4 && splits * chunk <= 24;
+    if (splits > 1) return !tile.pair && splits <= 8 && chunk <= 4 && splits * chunk < 24;
     return (chunk <= 2 && t32 <= 256) || (chunk <= 4 && t32 <= 8);
 }
 
@@ -2699,7 +2703,10 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
     // for a single pair); every other kernel one per partition.
     const bool direct128 = tile.bm == 128 && b_rows && (amode == KCD || a_rows);
     const bool paired = direct128 && tile.pair && splits >= 2 && reinterpret_cast<uintptr_t>(c) % 16 == 0;
-    if ((split_req == 0 || (splits > 1 && tile.bm == 64)) &&
+    // (unsplit: the 64x64 kernels are ahead with 16-byte loads of both operands,
+    // except over whole K-tiles of a k-contiguous A)
+    const bool small_loads = splits > 1 || !g.a_vec || !g.b_vec || (k % 32 == 0 && g.sak == 1);
+    if ((split_req == 0 || (splits > 1 && tile.bm == 64)) && small_loads &&
         small_fits(static_cast<uint32_t>(batch), m, n, splits, chunk, tile)) {
         g.tiles_m = ceil_div(m, 32u);
         g.tiles_n = ceil_div(n, 32u);
