@@ -383,7 +383,9 @@ def case_gemm(name, hip, ops, timer, rng, out):
     c = DeviceArray((m, n), np.float32)
     ms = time_batch(lambda i: ops.matmul(av, bv, out=c), timer, 10 if m * n * k > 2**36 else 20)
     peak, kernel = matrix_roof(lambda: ops.matmul(av, bv, out=c))
-    splits = 1 if peak == TRIPLE_PEAK_TFLOPS else ops.gemm_plan(1, m, n, k)[0]
+    splits = ops.gemm_plan(1, m, n, k)[0]
+    if splits == 2 and peak == TRIPLE_PEAK_TFLOPS:
+        splits = 1  # the 64x64 tile's two groups of stages
     tf = 2.0 * m * n * k / ms / 1e9
     out[name] = {"ms": round(ms, 5), "tflops": round(tf, 2), "kernel": kernel, "peak": peak,
                  "frac_of_peak": round(tf / peak, 4), "splits": splits}

@@ -520,9 +520,9 @@ int vkhip_sgd_step(const vkhip_sgd_param* params, size_t count, float lr, float 
 /* ======================================================================== */
 /* One choice the backend made, what it rejected, why, and the numbers that
  * forced it (reference vkml::observe::Decision, include/vkml/util/observe.h:
- * 55-93). Sites: "matmul.kernel", "matmul.split_k" (products on the fp32
- * matrix cores), "matmul.operands" (products as three bf16 terms; their kernels
- * are gemm_triple_<tile>, unsplit), "conv.input_grad", "reduce.structure",
+ * 55-93). Sites: "matmul.kernel", "matmul.split_k", "matmul.operands" (of
+ * products as three bf16 terms, whose kernels are gemm_triple_<tile> and which
+ * publish matmul.split_k only when split), "conv.input_grad", "reduce.structure",
  * "softmax.structure", "col2im.kernel", "max_pool2d.kernel",
  * "allocator.release". The strings live for the duration of the callback
  * only. `dispatch` names the unit of work the choice produced: the same id the

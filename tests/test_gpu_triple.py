@@ -226,20 +226,53 @@ def test_sums_of_one_term_are_rounded_as_in_fp32(hip):
     assert np.max(np.abs(got - exact) / exact) <= 2.0 ** -24 * (1 + 2.0 ** -7)
 
 
-@pytest.mark.parametrize("m,n,k", [(1024, 1024, 16384), (130, 780, 16400)])
-def test_split_plans_keep_their_partitions(hip, m, n, k):
-    """A product whose K the plan splits is summed partition by partition: long
-    chains of products of one sign lose more than the fp32 kernels do."""
-    assert ops.gemm_plan(1, m, n, k)[0] > 2
+# (128x128 and 256x128 tiles, ragged rows, a last stage of 4 and of 1 k; pairs of
+# partitions)
+@pytest.mark.parametrize("batch,m,n,k,terms", [(1, 336, 422, 20164, True), (1, 448, 691, 20308, True),
+                                               (4, 210, 446, 7473, True), (1, 304, 208, 34936, False)])
+@pytest.mark.parametrize("one_sign", [False, True])
+def test_split_plans_keep_their_partitions(hip, batch, m, n, k, terms, one_sign):
+    """A product whose K the plan splits is summed partition by partition, in
+    chains no longer than the fp32 kernels': no less exact than those, also
+    where every product is of one sign, in every layout the same bits."""
+    splits, chunk = ops.gemm_plan(batch, m, n, k)
+    assert splits > 2
     rng = np.random.default_rng(SEED + 7)
-    a, b = (np.maximum(rng.standard_normal(s), 0).astype(np.float32) for s in ((m, k), (k, n)))
+    lead = (batch,) if batch > 1 else ()
+    a, b = (rng.standard_normal(lead + s).astype(np.float32) for s in ((m, k), (k, n)))
+    if one_sign:
+        a, b = np.maximum(a, 0), np.maximum(b, 0)
     with DecisionRecorder() as rec:
         got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
-    assert _operand_kinds(rec) == []
+    assert _operand_kinds(rec) == ["three_bf16_terms"] * terms
+    assert [d["chose"] for d in rec.decisions if d["site"] == "matmul.split_k"] == [f"split_k_{splits}"]
     rows = np.arange(0, m, 16)
-    fp32 = ops.matmul(_view(a, "n"), _view(b, "n"), kernel=_lib.GEMM_MFMA).numpy()[rows]
-    exact = a[rows].astype(np.float64) @ b.astype(np.float64)
-    assert _off(got[rows], exact) <= _off(fp32, exact)
+    fp32 = ops.matmul(_view(a, "n"), _view(b, "n"), kernel=_lib.GEMM_MFMA).numpy()[..., rows, :]
+    exact = a[..., rows, :].astype(np.float64) @ b.astype(np.float64)
+    assert _off(got[..., rows, :], exact) <= _off(fp32, exact)
+    for la, lb in (("n", "t"), ("t", "n"), ("o", "o"), ("r", "n")):
+        same = ops.matmul(_view(a, la), _view(b, lb)).numpy()
+        assert np.array_equal(same.view(np.uint32), got.view(np.uint32)), (la, lb)
+
+
+@pytest.mark.parametrize("n,c,hw,cout,window", [(70, 33, (24, 20), 250, 3), (40, 40, (24, 24), 200, 5)])
+def test_weight_gradients_summed_over_a_batch(hip, n, c, hw, cout, window):
+    """The batch folded into K, ragged rows and columns: each partition a chain,
+    and a fold that rounds log2(partitions) times."""
+    rng = np.random.default_rng(SEED + c)
+    x = rng.uniform(-1, 1, (n, c) + hw).astype(np.float32)
+    g = rng.standard_normal((n, cout) + hw).astype(np.float32)
+    k, ck = n * hw[0] * hw[1], c * window * window
+    splits, chunk = ops.gemm_plan(1, cout, ck, k)
+    dx, dg = DeviceArray.from_numpy(x), DeviceArray.from_numpy(g)
+    with DecisionRecorder() as rec:
+        got = ops.conv2d_weight_grad_sum(dx, dg, window, 1, window // 2).numpy()
+    assert _operand_kinds(rec) == ["three_bf16_terms"]
+    cols = ops.im2col(dx, window, 1, window // 2).numpy()
+    exact = np.zeros((cout, ck))
+    for image in range(n):
+        exact += g[image].reshape(cout, -1).astype(np.float64) @ cols[image].astype(np.float64).T
+    assert _off(got, exact) <= _bound(32 * chunk) + 2.0 ** -24 * np.sqrt(np.log2(splits))
 
 
 def test_tiny_inputs_among_ordinary_ones_change_nothing(hip):

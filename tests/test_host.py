@@ -451,7 +451,8 @@ def test_program_output_order_hoists_the_output_cone_within_hazards():
     ((1, 2100, 2300, 100), False),   # 18.7 21.4
     ((16, 576, 256, 256), False),    # 18.3 20.3
     ((20, 864, 256, 96), False),     # 15.7 20.6
-    ((1, 1024, 1024, 4096), False),  # 84 94, K split
+    ((1, 128, 576, 12288), False),   # 45.6 56.3, K split, few workgroups
+    ((1, 480, 756, 21632), True),    # 137.8 129.0, K split
     ((4, 496, 139, 1152), False),    # 20.8 23.1, fewer tiles than CUs
     ((32, 288, 560, 123), True),     # 35.2 23.5
     ((16, 1872, 448, 118), True),    # 61.1 41.4

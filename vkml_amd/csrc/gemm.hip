@@ -2284,9 +2284,11 @@ int gemm_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k, int32_t split_
 }
 
 // ---- products on the bf16 matrix cores (gemm_triple.h) --------------------------
-// The tile of an AUTO product that runs there.
+// The tile of a product that runs there, and its partitions: `slices` of
+// `chunk` K-tiles.
 struct TriplePlan {
     int tile = -1;  // kTripleTiles; negative: the fp32 matrix cores
+    uint32_t slices = 1, chunk = 0;
     explicit operator bool() const { return tile >= 0; }
 };
 
@@ -2318,6 +2320,37 @@ static const TileTime kFp32Tiles[] = {{64, 64, 4.9, 0.53, 0.0, 0.92, 6.2e-7, ""}
 // and 9.8 here; 660^3, 2.9e8, 16.5 and 16.3).
 constexpr double kTripleMinMacs = 3e8;
 
+// The plan of a product whose K the fp32 plan splits: the same partitions, so
+// that no chain of products is longer than there (as chains of two or three
+// partitions the terms were less exact where every product is of one sign:
+// relu(N) against relu(N), 1024x1024x16384, 1.64e-7 of the result, fp32
+// 1.30e-7), each a workgroup of a 128-row tile. Where those fill three quarters
+// of the CUs, with enough K-tiles each, they take 0.46 to 1.01 of the fp32 time
+// (1401x384x25864 226 -> 212 us, 784x526x6156 113 -> 69, the weight gradient
+// [64,192,32,32] -> 256 457 -> 337), with less than two thirds of the CUs 1.0
+// to 2.2 of it. Enough is eight K-tiles for gathered and 4-byte loads, twelve
+// against the fp32 kernels' 16-byte loads (9: 128x784x16384 TN 38.2 -> 40.6).
+static TriplePlan triple_split_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k, uint32_t splits, uint32_t chunk,
+                                    uint32_t least_chunk) {
+    TriplePlan best;
+    if (m <= 64 || n <= 64 || chunk < least_chunk) return best;
+    if (static_cast<double>(batch) * m * n * k < kTripleMinMacs) return best;
+    const double cus = ctx().ready ? ctx().caps.compute_units : 256.0;
+    const double partials = static_cast<double>(batch) * m * n * splits;
+    double best_us = 1e30;
+    for (int tile = 1; tile < 3; ++tile) {
+        const TileTime& tt = kTripleTiles[tile];
+        const uint64_t wgs = static_cast<uint64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch * splits;
+        if (tile == 1 && static_cast<double>(wgs) < 0.75 * cus) break;
+        const double us = tt.us(wgs, std::min(ceil_div(k, 16u), 2 * chunk), partials, cus);
+        if (us < best_us) {
+            best_us = us;
+            best = TriplePlan{tile, splits, chunk};
+        }
+    }
+    return best;
+}
+
 // A product takes the three terms where their time is below the fp32 kernels'
 // by the model, by 8%, or within 10% of it for sizes that are not multiples of
 // four, whose fp32 loads are 4 bytes wide (3808x960x6145 758 us on the fp32
@@ -2329,27 +2362,26 @@ constexpr double kTripleMinMacs = 3e8;
 // workgroup there waits for its own loads, [16,64,20,20] -> 128 5x5 input
 // gradient 59 us on the fp32 cores and 79 here, 4 of 496x139x1152 21 and 23.
 //
-// Nor for a product whose K the fp32 plan splits. Its partitions are short
-// chains, added up at the end: as long chains the three terms were less exact
-// where every product is of one sign (relu(N) against relu(N), 1024x1024x16384
-// 1.64e-7 of the result, fp32 1.30e-7), and as short ones no faster
-// (1024x1024x4096 94 us, fp32 84; 256x256x65536 97 and 85; 128x784x16384 49 and
-// 44). Two partitions of one round of 64x64 tiles are the exception, since the
-// two groups of stages of the 64x64 tile are two such chains: 1024^3 25.4 us,
-// fp32 33.7 with B transposed and 24.7 without.
-static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k) {
+// Two partitions of one round of 64x64 tiles are the two groups of stages of
+// the 64x64 tile: 1024^3 25.4 us, fp32 33.7 with B transposed and 24.7 without.
+//
+// gathered: a convolution that need not have the lowered product's bits, where
+// the fp32 kernels' gathers take an eighth more than their loads: within 10%.
+static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k, bool gathered = false) {
     TriplePlan best;
     if (m <= 32 || n <= 32 || k < 64) return best;
     if (static_cast<double>(batch) * m * n * k < kTripleMinMacs) return best;
     uint32_t splits, chunk;
     TileChoice plan;
     gemm_plan(batch, m, n, k, 0, splits, chunk, plan, true);
-    if (splits > 2 || (splits == 2 && plan.bm != 64)) return best;
+    const bool ragged = m % 4 != 0 || n % 4 != 0 || k % 4 != 0;
+    // (pairs of partitions write half the partials that these would)
+    if (splits > 2 || (splits == 2 && plan.bm != 64))
+        return plan.pair ? best : triple_split_plan(batch, m, n, k, splits, chunk, ragged ? 8 : 12);
     const double cus = ctx().ready ? ctx().caps.compute_units : 256.0;
     const double out_elems = static_cast<double>(batch) * m * n;
     const TileTime& fp32 = kFp32Tiles[plan.bm == 128];
-    const bool ragged = m % 4 != 0 || n % 4 != 0 || k % 4 != 0;
-    double below = (ragged ? 1.1 : 0.92) * fp32.us(plan.tiles, ceil_div(k, 32u), out_elems, cus);
+    double below = (ragged || gathered ? 1.1 : 0.92) * fp32.us(plan.tiles, ceil_div(k, 32u), out_elems, cus);
     if (splits == 2) below = 1e30;
     for (int tile = 0; tile < (splits == 1 ? 3 : 1); ++tile) {
         const TileTime& tt = kTripleTiles[tile];
@@ -2358,7 +2390,7 @@ static TriplePlan triple_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k
         const double us = tt.us(tiles, ceil_div(k, 16u), out_elems, cus);
         if (us < below) {
             below = us;
-            best.tile = tile;
+            best = TriplePlan{tile, 1, ceil_div(k, 32u)};
         }
     }
     return best;
@@ -2370,7 +2402,12 @@ static void publish_triple(const char* op, const TriplePlan& t, const char* inst
     const TileTime& tt = kTripleTiles[t.tile];
     const char* because = "the three-term time is below the fp32 kernels'";
     publish("matmul.kernel", op, tt.name, instead, because,
-            static_cast<int64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch, ctx().ready ? ctx().caps.compute_units : 256);
+            static_cast<int64_t>(ceil_div(m, tt.bm)) * ceil_div(n, tt.bn) * batch * t.slices, ctx().ready ? ctx().caps.compute_units : 256);
+    if (t.slices > 1) {
+        char chose[32];
+        snprintf(chose, sizeof chose, "split_k_%u", t.slices);
+        publish("matmul.split_k", op, chose, "unsplit", "the partitions of the fp32 plan", t.slices, t.chunk);
+    }
     publish("matmul.operands", op, "three_bf16_terms", "fp32", because, m, n);
 }
 
@@ -2379,10 +2416,11 @@ static void publish_triple(const char* op, const TriplePlan& t, const char* inst
 static int launch_triple_product(GemmArgs& g, const Im2colB& im, const TriplePlan& t, uint32_t batch, int am, int bm) {
     g.tiles_m = ceil_div(g.m, kTripleTiles[t.tile].bm);
     g.tiles_n = ceil_div(g.n, kTripleTiles[t.tile].bn);
-    g.flat_splits = 0;
-    const uint64_t tiles = static_cast<uint64_t>(g.tiles_m) * g.tiles_n;
-    if (tiles > 0x7fffffffull) return fail(VKHIP_ERR_UNSUPPORTED, "gemm: %llu workgroups", static_cast<unsigned long long>(tiles));
-    const dim3 grid(static_cast<uint32_t>(tiles), 1, batch);
+    g.chunk = t.chunk;
+    const uint64_t wgs = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * t.slices;
+    if (wgs > 0x7fffffffull) return fail(VKHIP_ERR_UNSUPPORTED, "gemm: %llu workgroups", static_cast<unsigned long long>(wgs));
+    g.flat_splits = t.slices > 1 ? t.slices : 0;
+    const dim3 grid(static_cast<uint32_t>(wgs), 1, batch);
     return t.tile == 0   ? launch_triple_64x64(g, im, grid, am, bm)
            : t.tile == 1 ? launch_triple_128x128(g, im, grid, am, bm)
                          : launch_triple_256x128(g, im, grid, am, bm);
@@ -2668,10 +2706,18 @@ static int gemm_core(const float* a, const vkhip_operand& ad, const float* b, co
 
     const uint64_t out_elems = batch * m * n;
     if (triple) {
-        g.c = c;  // (an epilogue follows as a pass of its own)
+        g.c = c;
+        if (triple.slices > 1) {
+            const int st = partials(out_elems * triple.slices * sizeof(float), &g.c);
+            if (st != VKHIP_OK) return st;
+            g.split_stride = out_elems;
+        }
         int am = triple_mode(m, k, g.sam, g.sak), bm = triple_mode(n, k, g.sbn, g.sbk);
         if (am == TG || bm == TG) am = bm = TG;
-        return launch_triple_product(g, Im2colB{}, triple, static_cast<uint32_t>(batch), am, bm);
+        const int st = launch_triple_product(g, Im2colB{}, triple, static_cast<uint32_t>(batch), am, bm);
+        if (st != VKHIP_OK || triple.slices == 1) return st;  // (an epilogue follows as a pass of its own)
+        *fused = true;
+        return launch_split_k_reduce(g.c, c, out_elems, triple.slices, fe);
     }
     int amode = akc ? (g.a_vec ? KCV : KCS) : (g.a_vec ? RCV : RCS);
     // The buffer-load paths (straight-to-LDS operands and the direct kernels)
@@ -3504,7 +3550,7 @@ static int launch_conv_wgrad_stream(SmallConvFwd p, const float* gr, const vkhip
 
 int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
                    const vkhip_operand& wd, float* out, const vkhip_unfold& p, const float* bias,
-                   int64_t bias_stride, bool relu, bool terms) {
+                   int64_t bias_stride, bool relu, bool terms, bool lowered) {
     if (p.kernel_h <= 0 || p.kernel_w <= 0 || p.stride_h <= 0 || p.stride_w <= 0 ||
         p.dilation_h <= 0 || p.dilation_w <= 0 || p.pad_h < 0 || p.pad_w < 0)
         return fail(VKHIP_ERR_INVALID, "conv2d: invalid window geometry");
@@ -3567,9 +3613,9 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
     TileChoice tile;
     gemm_plan(static_cast<uint32_t>(batch), m, n, k, 0, splits, chunk, tile);
     const bool weight_rows = triple_mode(m, k, wd.nb[2], 1) == TK;
-    // the plan gemm() takes for the same product, so the same bits
+    // lowered: the plan gemm() takes for the same product, so the same bits
     const TriplePlan triple = terms && !bias && !relu && weight_rows
-                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k) : TriplePlan{};
+                                  ? triple_plan(static_cast<uint32_t>(batch), m, n, k, !lowered) : TriplePlan{};
     const char* const fp32_kernel = tile.bm == 128 ? "gemm_mfma_128x128_implicit_im2col"
                                                    : "gemm_mfma_64x64_implicit_im2col";
     if (triple)
@@ -3613,7 +3659,7 @@ int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
 
     const uint64_t out_elems = batch * m * n;
     float* target = out;
-    if (triple) splits = 1;
+    if (triple) splits = triple.slices;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -3785,7 +3831,7 @@ int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
     const int amode = a_kcd ? KCD : (g.a_vec ? KCV : KCS);
     const uint64_t out_elems = batch * m * n;
     float* target = out;
-    if (triple) splits = 1;
+    if (triple) splits = triple.slices;
     if (splits > 1) {
         float* ws = nullptr;
         int st = workspace(out_elems * splits * sizeof(float), &ws);
@@ -4027,10 +4073,18 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     uint32_t splits, chunk;
     TileChoice tile;
     gemm_plan(1, m, n, k, 0, splits, chunk, tile, true);
-    publish("matmul.kernel", "conv2d_weight_grad_sum",
-            tile.bm == 128 ? "gemm_mfma_128x128_batch_folded" : "gemm_mfma_64x64_batch_folded",
-            "per_image_products_then_batch_sum", "the batch folded into K: one product, no intermediate",
-            static_cast<int64_t>(tile.tiles), static_cast<int64_t>(splits));
+    const TriplePlan triple = terms && gd.nb[1] >= 0 && triple_image_fits(im, oh) &&
+                                      triple_mode(m, static_cast<uint32_t>(L), gd.nb[2], 1) == TK
+                                  ? triple_split_plan(1, m, n, k, splits, chunk, 8) : TriplePlan{};
+    const char* const fp32_kernel = tile.bm == 128 ? "gemm_mfma_128x128_batch_folded" : "gemm_mfma_64x64_batch_folded";
+    if (triple) {
+        splits = triple.slices;
+        publish_triple("conv2d_weight_grad_sum", triple, fp32_kernel, 1, m, n);
+    } else {
+        publish("matmul.kernel", "conv2d_weight_grad_sum", fp32_kernel, "per_image_products_then_batch_sum",
+                "the batch folded into K: one product, no intermediate", static_cast<int64_t>(tile.tiles),
+                static_cast<int64_t>(splits));
+    }
     im.x = x;
     im.sn = xd.nb[0];
     im.L = static_cast<uint32_t>(L);
@@ -4064,7 +4118,9 @@ int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float*
     g.c = target;
     g.split_stride = splits > 1 ? out_elems : 0;
     int st;
-    if (tile.bm == 128 && wgrad_direct_fits(g, static_cast<uint32_t>(L), target)) {
+    if (triple) {
+        st = launch_triple_product(g, im, triple, 1, TKB, TTB);
+    } else if (tile.bm == 128 && wgrad_direct_fits(g, static_cast<uint32_t>(L), target)) {
         const bool narrow = wgrad_narrow_tiles(g, splits, 1);
         if (narrow) g.tiles_n = ceil_div(n, 64u);
         const uint64_t flat = static_cast<uint64_t>(g.tiles_m) * g.tiles_n * splits;
@@ -4187,7 +4243,7 @@ int conv2d_input_grad(const float* gr, const vkhip_operand& gd, const float* w, 
         wd.nb[1] = 0;
         wd.nb[2] = static_cast<int64_t>(cout) * kk;
         wd.nb[3] = 1;
-        return conv2d_forward(gr, gd, wt, wd, out, q, nullptr, 0, false, terms);
+        return conv2d_forward(gr, gd, wt, wd, out, q, nullptr, 0, false, terms, false);
     }
     if (ck > 0xffffffffull || L > 0xffffffffull)
         return fail(VKHIP_ERR_UNSUPPORTED, "conv2d input grad: extents too large");
@@ -4284,7 +4340,7 @@ extern "C" int vkhip_conv2d(const float* x, const vkhip_operand* x_desc, const f
     if (st != VKHIP_OK) return st;
     vkhip::Unit unit("conv2d");
     if (!x_desc || !w_desc || !p) return vkhip::fail(VKHIP_ERR_INVALID, "conv2d: null argument");
-    return vkhip::conv2d_forward(x, *x_desc, w, *w_desc, out, *p, nullptr, 0, false, true);
+    return vkhip::conv2d_forward(x, *x_desc, w, *w_desc, out, *p, nullptr, 0, false, true, true);
 }
 
 extern "C" int vkhip_conv2d_weight_grad(const float* x, const vkhip_operand* x_desc,

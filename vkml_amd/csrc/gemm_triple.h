@@ -80,10 +80,13 @@ __device__ __forceinline__ __attribute__((address_space(3))) V& lds_at(Lds p) {
 //   TK   unit k stride: groups of four k, 16-byte loads at any float address.
 //   TR   unit row stride: four rows of one k, 16-byte loads along the rows.
 //   TG   any strides: 4-byte loads.
-//   TI   B gathered from the image (IMG), TT its transpose (IMGT).
-enum TripleMode { TK = 0, TR, TG, TI, TT };
+//   TKB  TK with the batch folded into K (conv weight gradient summed over
+//        the batch: k = image * L + position, L a multiple of 32).
+//   TI   B gathered from the image (IMG), TT its transpose (IMGT), TTB the
+//        transpose with the batch folded into K (IMGTB).
+enum TripleMode { TK = 0, TR, TG, TKB, TI, TT, TTB };
 // Modes whose planes are k rows of R values (the others': rows of 16 k).
-constexpr bool triple_k_rows(int mode) { return mode == TR || mode == TT; }
+constexpr bool triple_k_rows(int mode) { return mode == TR || mode == TT || mode == TTB; }
 
 constexpr uint32_t kTripleTiny = 0x11000000u - 1u;  // 2 * bits(2^-110) - 1
 
@@ -127,12 +130,12 @@ struct TripleOperand {
     static constexpr int NG = R * 16 / T / 4;
     static_assert(NG >= 1, "at least one group of four per thread");
     static constexpr uint32_t kBytes = 3 * R * 32, kBytes32 = R * kTriplePitch32 * 4;  // of a stage
-    static constexpr bool KMAP = MODE == TK || MODE == TG;
+    static constexpr bool KMAP = MODE == TK || MODE == TKB || MODE == TG;
 
     const char* base;  // this batch's operand
     int64_t s_k;
     uint32_t kdim;
-    uint32_t voff[MODE == TK || MODE == TR ? NG : 1];
+    uint32_t voff[MODE == TK || MODE == TKB || MODE == TR ? NG : 1];
     int64_t goff[MODE == TG ? NG : 1];
     uint32_t slot;
     // TI: a lane has one position for all its groups, a wave's k are the same
@@ -145,8 +148,9 @@ struct TripleOperand {
     uint32_t out_lo, out_hi;  // bit r: window element r of the position is padding
     // TT: a lane has one position per stage and four window rows per group, so
     // that a load of 64 lanes covers 16 consecutive positions of four rows.
-    int32_t off4[MODE == TT ? 4 * NG : 1];     // a row's byte offset
-    uint32_t disp[MODE == TT ? 4 * NG : 1];    // and displacement: h, and w << 16
+    static constexpr bool IMAGE_T = MODE == TT || MODE == TTB;
+    int32_t off4[IMAGE_T ? 4 * NG : 1];     // a row's byte offset
+    uint32_t disp[IMAGE_T ? 4 * NG : 1];    // and displacement: h, and w << 16
 
     // (row, k group of four) of group i, for the modes that hold such groups
     __device__ __forceinline__ static void row_kq(int t, int i, int& r, int& kq) {
@@ -161,8 +165,8 @@ struct TripleOperand {
     // Modes with k rows: group i is one k of rows quad(i) .. + 3. TR: lanes
     // along the rows, TT: along k.
     static constexpr int KSTEP = 4 * T / R, QSTEP = T / 4;
-    __device__ __forceinline__ static int quad_k(int t, int i) { return MODE == TT ? t & 15 : t / (R / 4) + i * KSTEP; }
-    __device__ __forceinline__ static int quad(int t, int i) { return MODE == TT ? (t >> 4) * 4 + i * QSTEP : 4 * (t % (R / 4)); }
+    __device__ __forceinline__ static int quad_k(int t, int i) { return IMAGE_T ? t & 15 : t / (R / 4) + i * KSTEP; }
+    __device__ __forceinline__ static int quad(int t, int i) { return IMAGE_T ? (t >> 4) * 4 + i * QSTEP : 4 * (t % (R / 4)); }
 
     // The operand's row that the tile's row x (counted from the operand's
     // start) holds, and whether the output has it. TR loads four rows at a
@@ -189,7 +193,7 @@ struct TripleOperand {
 #pragma unroll
             for (int i = 0; i < NG; ++i) voff[i] = (static_cast<uint32_t>(quad_k(t, i) * sk) + rb) * 4u;
             slot = triple_slot_t<R>(quad(t, 0), quad_k(t, 0));
-        } else if constexpr (MODE == TT) {
+        } else if constexpr (IMAGE_T) {
             slot = triple_slot_t<R>(quad(t, 0), quad_k(t, 0));
 #pragma unroll
             for (int i = 0; i < 4 * NG; ++i) {
@@ -205,7 +209,7 @@ struct TripleOperand {
             int r, kq;
             row_kq(t, 0, r, kq);
             slot = triple_slot(r, kq >> 1) + ((kq & 1) << 3);
-            if constexpr (MODE == TK || MODE == TG) {
+            if constexpr (MODE == TK || MODE == TKB || MODE == TG) {
 #pragma unroll
                 for (int i = 0; i < NG; ++i) {
                     row_kq(t, i, r, kq);
@@ -245,6 +249,11 @@ struct TripleOperand {
                         v[i][j] = k + j < kdim ? *reinterpret_cast<const float*>(p + voff[i] + 4 * j) : 0.0f;
                 }
             }
+        } else if constexpr (MODE == TKB) {
+            const uint32_t n = im.div_L.div(k0);
+            const char* p = base + (static_cast<int64_t>(n) * s_k + (k0 - n * im.L)) * 4;  // s_k: image stride
+#pragma unroll
+            for (int i = 0; i < NG; ++i) v[i] = *reinterpret_cast<const f32x4u*>(p + voff[i]);
         } else if constexpr (MODE == TR) {
             const char* p = base + static_cast<int64_t>(k0) * s_k * 4;
 #pragma unroll
@@ -279,9 +288,16 @@ struct TripleOperand {
                                    img, static_cast<int32_t>((pad & 0x80000000u) | lane4), tab[e], 0));
                 }
         } else {
-            const uint32_t p = k0 + quad_k(t, 0);
+            uint32_t p = k0 + quad_k(t, 0), positions = kdim;
+            const char* image = base;
+            if constexpr (MODE == TTB) {
+                const uint32_t n = im.div_L.div(k0);
+                image += static_cast<int64_t>(n) * im.sn * 4;
+                p -= n * im.L;
+                positions = im.L;
+            }
             const __amdgpu_buffer_rsrc_t img = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<char*>(base), 0, static_cast<int32_t>(0x80000000u), 0x00020000);
+                const_cast<char*>(image), 0, static_cast<int32_t>(0x80000000u), 0x00020000);
             const uint32_t oh = im.div_ow.div(p), ow = p - oh * static_cast<uint32_t>(im.ow);
             const int32_t h0 = static_cast<int32_t>(oh) * im.strh - im.padh;
             const int32_t w0 = static_cast<int32_t>(ow) * im.strw - im.padw;
@@ -290,7 +306,7 @@ struct TripleOperand {
             // lesser of (h, w) and (H - 1, W - 1), unsigned, is (h, w); a
             // position past K lies outside every image
             typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-            const u16x2 origin = {static_cast<uint16_t>(p < kdim ? h0 : 0x6000), static_cast<uint16_t>(w0)};
+            const u16x2 origin = {static_cast<uint16_t>(p < positions ? h0 : 0x6000), static_cast<uint16_t>(w0)};
             const u16x2 last = {static_cast<uint16_t>(im.H - 1), static_cast<uint16_t>(im.W - 1)};
 #pragma unroll
             for (int i = 0; i < 4 * NG; ++i) {
@@ -312,7 +328,7 @@ struct TripleOperand {
             // group i: KSTEP k or QSTEP rows further on, T / 4 rows further on,
             // or another k group
             const Lds p = MODE == TR   ? lds + slot + i * (KSTEP * 2 * R)
-                          : MODE == TT    ? lds + (slot ^ (i * (QSTEP * 2)))
+                          : IMAGE_T    ? lds + (slot ^ (i * (QSTEP * 2)))
                           : KMAP       ? lds + slot + i * (T / 4 * 32)
                                        : lds + (slot ^ (i * (8 * T / R)));
             static_assert(MODE != TR || NG == 1 || KSTEP % 8 == 0, "the exchanges repeat every eight k");
@@ -334,7 +350,7 @@ struct TripleOperand {
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
             if constexpr (triple_k_rows(MODE)) {
-                const uint32_t step = MODE == TT ? QSTEP * (kTriplePitch32 * 4) : KSTEP * 4;
+                const uint32_t step = IMAGE_T ? QSTEP * (kTriplePitch32 * 4) : KSTEP * 4;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) lds_at<float>(lds + slot32 + i * step + j * (kTriplePitch32 * 4)) = v[i][j];
             } else {
@@ -420,9 +436,9 @@ struct TripleTile {
     f32x16 acc[MI][NI], cor[MI][NI];  // the hh' products; the smaller ones
     TripleReads<AM, BM, MI> ra;
     TripleReads<BMODE, BN, NI> rb;
-    uint32_t full;        // whole stages
+    uint32_t kt0, full;   // this partition's first stage, and the end of its whole stages
     int kg, ns, mine;     // whole stages of the longest group, and of this one
-    bool tail;            // K ends inside another one
+    bool tail;            // K ends inside the partition's last stage
 
     __device__ __forceinline__ void zero() {
 #pragma unroll
@@ -441,7 +457,7 @@ struct TripleTile {
                 for (int r = 0; r < 16; ++r) acc[i][j][r] += cor[i][j][r];
     }
     // The whole stage that is this group's s-th, or the last whole one.
-    __device__ __forceinline__ uint32_t stage_of(int s) const { return min(kg + s * KG, full - 1u); }
+    __device__ __forceinline__ uint32_t stage_of(int s) const { return min(kt0 + kg + s * KG, full - 1u); }
 
     // One stage's products; `next` (staging of the next stage) is called where
     // it can run beside them.
@@ -565,16 +581,20 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
     const int wm0 = (wave / (BN / WN)) * WM, wn0 = (wave % (BN / WN)) * WN;
     const int lrow = lane & 31, kh = lane >> 5;
 
-    uint32_t tm, tn, split;  // one partition: split is 0
+    uint32_t tm, tn, split;
     tile_of(g, tm, tn, split);
     const uint32_t row0 = tm * BM, col0 = tn * BN;
     const uint32_t z = blockIdx.z, i0 = z / g.b1, i1 = z % g.b1;
 
     Tile tile;
     tile.kg = kg;
-    tile.full = g.k / 16u;
-    tile.tail = g.k % 16u != 0;
-    const int whole = static_cast<int>(tile.full);
+    tile.kt0 = split * 2u * g.chunk;
+    const uint32_t kt1 = min((g.k + 15u) / 16u, tile.kt0 + 2u * g.chunk);
+    tile.full = min(kt1, g.k / 16u);
+    tile.tail = kt1 > tile.full;
+    // (a partition of a tail alone has no whole stage: its prefetches read the
+    // stage before it)
+    const int whole = static_cast<int>(tile.full - tile.kt0);
     tile.ns = (whole + KG - 1) / KG;
     tile.mine = (whole - kg + KG - 1) / KG;
     tile.ra.init(0, wm0, lane);
@@ -583,8 +603,8 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
 
     TripleStager<OA, OB, D> st;
     st.t = wave * 64 + lane;
-    st.a.init(g.a + i0 * g.sa0 + i1 * g.sa1, g.sam, g.sak, row0, g.m, g.k, im, st.t);
-    st.b.init(BMODE >= TI ? im.x + static_cast<int64_t>(z) * im.sn
+    st.a.init(g.a + i0 * g.sa0 + i1 * g.sa1, g.sam, AM == TKB ? g.sa1 : g.sak, row0, g.m, g.k, im, st.t);
+    st.b.init(BMODE >= TI ? im.x + (BMODE == TTB ? 0 : static_cast<int64_t>(z) * im.sn)
                           : g.b + i0 * g.sb0 + i1 * g.sb1,
               g.sbn, g.sbk, col0, g.n, g.k, im, st.t);
     uint32_t tiny = ~0u;
@@ -647,7 +667,7 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
     }
 
     // register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32
-    float* cbase = g.c + static_cast<uint64_t>(z) * g.m * g.n;
+    float* cbase = g.c + static_cast<uint64_t>(split) * g.split_stride + static_cast<uint64_t>(z) * g.m * g.n;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -659,8 +679,8 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64 * KG, OCC) void gemm_tripl
                 uint32_t row;
                 if (OA::real_row(row0 + wm0 + 32 * i + 8 * (r / 4) + 4 * kh + (r % 4), g.m, row) && col_in) {
                     float* at = cbase + static_cast<uint64_t>(row) * g.n + col;
-                    // outputs of large tiles and convolutions are read by
-                    // later kernels only
+                    // outputs of large tiles and convolutions, and split-K
+                    // partials, are read by later kernels only
                     if constexpr (BM >= 128 || BMODE >= TI)
                         __builtin_nontemporal_store(acc[i][j][r], at);
                     else
@@ -685,7 +705,7 @@ int launch_triple(const GemmArgs& g, const Im2colB& im, dim3 grid, int am, int b
     constexpr int threads = BM / WM * (BN / WN) * 64 * KG;
 #define VKHIP_TRIPLE(A, B)                                                                                   \
     if (am == A && bm == B) {                                                                                \
-        hipLaunchKernelGGL((gemm_triple_kernel<BM, BN, WM, WN, KG, D, (B == TT ? OCC_T : OCC), A, B>), \
+        hipLaunchKernelGGL((gemm_triple_kernel<BM, BN, WM, WN, KG, D, (B >= TT ? OCC_T : OCC), A, B>), \
                            grid, dim3(threads), 0, ctx().stream, g, im);                                     \
         VKHIP_LAUNCH_CHECK();                                                                                \
         return VKHIP_OK;                                                                                     \
@@ -697,6 +717,7 @@ int launch_triple(const GemmArgs& g, const Im2colB& im, dim3 grid, int am, int b
     VKHIP_TRIPLE(TG, TG)
     VKHIP_TRIPLE(TK, TI)
     VKHIP_TRIPLE(TK, TT)
+    VKHIP_TRIPLE(TKB, TTB)
 #undef VKHIP_TRIPLE
     return fail(VKHIP_ERR_INVALID, "gemm_triple: no kernel for operand modes %d, %d", am, bm);
 }

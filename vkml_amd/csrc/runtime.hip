@@ -20,10 +20,11 @@ namespace vkhip {
 int launch_im2col(const float* src, const vkhip_operand& sd, float* dst, const vkhip_unfold& p);
 int launch_col2im(const float* cols, float* dst, uint32_t n, uint32_t channels,
                   const vkhip_unfold& p);
-// (terms: as gemm()'s; a node passes false)
+// (terms: as gemm()'s; a node passes false. lowered: the bits of the product of
+// the columns)
 int conv2d_forward(const float* x, const vkhip_operand& xd, const float* w,
                    const vkhip_operand& wd, float* out, const vkhip_unfold& p, const float* bias,
-                   int64_t bias_stride, bool relu, bool terms);
+                   int64_t bias_stride, bool relu, bool terms, bool lowered);
 int conv2d_weight_grad(const float* x, const vkhip_operand& xd, const float* gr,
                        const vkhip_operand& gd, float* out, const vkhip_unfold& p, bool terms);
 int conv2d_weight_grad_sum(const float* x, const vkhip_operand& xd, const float* gr,
@@ -727,7 +728,7 @@ static int compute_node(const vkhip_node& nd) {
                                   static_cast<const float*>(w.data), wd,
                                   static_cast<float*>(nd.out.data), p,
                                   fused ? static_cast<const float*>(nd.src[2].data) : nullptr,
-                                  fused ? nd.src[2].nb[0] : 0, fused, false);
+                                  fused ? nd.src[2].nb[0] : 0, fused, false, true);
         }
         case VKHIP_OP_CONV2D_WEIGHT_GRAD: {
             vkhip_unfold p;

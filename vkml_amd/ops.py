@@ -40,8 +40,8 @@ def _f32(x: DeviceArray, what: str) -> None:
 
 def gemm_plan(batch: int, m: int, n: int, k: int, split_k: int = 0) -> tuple[int, int]:
     """(splits, chunk) of the fp32 kernels' plan under AUTO (or a forced request).
-    A product that matmul runs as three bf16 terms takes its K in one piece,
-    whatever this says (1, or 2 for one round of 64x64 tiles)."""
+    A product that matmul runs as three bf16 terms has the same partitions,
+    but for one round of 64x64 tiles (2 here), whose K it takes in one piece."""
     lib = _lib.load()
     s, c = c_uint32(), c_uint32()
     check(lib.vkhip_gemm_plan(batch, m, n, k, split_k, byref(s), byref(c)), "gemm_plan")
