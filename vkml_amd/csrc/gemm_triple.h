@@ -25,7 +25,7 @@
 // of it. All such inputs together change an output by at most K 2^-133 of the
 // largest input, so a workgroup that has staged one reads its operands again for
 // that and runs again only where an output is below K 2^-103 of it, 2^30 times
-// as much. (4096^3 on one box: 0.87 ms; with such an input in every tile, a
+// as much. (4096^3 on one card: 0.87 ms; with such an input in every tile, a
 // probability of 1e-34 among ordinary ones, 1.12, and 2.36 with a second pass
 // for all of them; 0.93 on the fp32 matrix cores.)
 //
@@ -55,7 +55,9 @@
 // CU, 120 us; 126) 50%, at 1024^3 22%: a stage of the 128x128 tile reads 72 KB
 // and writes 24 KB of LDS for 1024 cycles of MFMAs, of the 64x64 tile half of
 // that for a quarter of the MFMAs. The 128x128 tile's 128 registers, for two
-// workgroups per CU, spill up to seven values around the loop, none inside it.
+// workgroups per CU, spill up to three values around the loop, none inside it;
+// with both operands transposed fifteen, of which a stage reads one (2048^3 128
+// us; 116 to 129 in the other layouts).
 #pragma once
 
 #include <algorithm>
