@@ -2327,9 +2327,10 @@ constexpr double kTripleMinMacs = 3e8;
 // 1.30e-7), each a workgroup of a 128-row tile. Where those fill three quarters
 // of the CUs, with enough K-tiles each, they take 0.46 to 1.01 of the fp32 time
 // (1401x384x25864 226 -> 212 us, 784x526x6156 113 -> 69, the weight gradient
-// [64,192,32,32] -> 256 457 -> 337), with less than two thirds of the CUs 1.0
-// to 2.2 of it. Enough is eight K-tiles for gathered and 4-byte loads, twelve
-// against the fp32 kernels' 16-byte loads (9: 128x784x16384 TN 38.2 -> 40.6).
+// [48,192,32,32] -> 256 3x3 457 -> 337), with less than two thirds of the CUs
+// 0.7 to 2.2 of it, mostly above 1. Enough is eight K-tiles for gathered and
+// 4-byte loads, twelve against the fp32 kernels' 16-byte loads (9:
+// 128x784x16384 TN 38.2 -> 40.6).
 static TriplePlan triple_split_plan(uint32_t batch, uint32_t m, uint32_t n, uint32_t k, uint32_t splits, uint32_t chunk,
                                     uint32_t least_chunk) {
     TriplePlan best;
