@@ -83,7 +83,27 @@ def test_layouts_and_edges(hip, tile, batch, m, n, k):
         assert differ == 0, (la, lb)
 
 
-@pytest.mark.parametrize("m,n,k", [(1000, 1501, 777), (4099, 3841, 89)])
+# the same of sizes that the plan leaves to the fp32 kernels: K split, few tiles
+@pytest.mark.parametrize("batch,m,n,k", [(1, 257, 2049, 1025), (1, 67, 130, 40001), (1, 33, 4100, 2100),
+                                         (16, 129, 131, 1040)])
+def test_layouts_and_edges_of_fp32_products(hip, batch, m, n, k):
+    rng = np.random.default_rng(SEED + m + n + k)
+    lead = (batch,) if batch > 1 else ()
+    a = rng.standard_normal(lead + (m, k), dtype=np.float32)
+    b = rng.standard_normal(lead + (k, n), dtype=np.float32)
+    print(f"fp32 {batch} {m}x{n}x{k}", flush=True)
+    with DecisionRecorder() as rec:
+        got = ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
+    assert _operand_kinds(rec) == []
+    rows = np.unique(np.r_[0:4, m // 2, m - 4:m])
+    exact = a[..., rows, :].astype(np.float64) @ b.astype(np.float64)
+    assert normwise_rel_err(got[..., rows, :], exact) <= min(gemm_tolerance(k), 2.0 ** -23 * np.sqrt(k))
+    for la, lb in (("n", "t"), ("t", "n"), ("t", "t"), ("o", "o"), ("r", "n"), ("n", "r")):
+        same = ops.matmul(_view(a, la), _view(b, lb)).numpy()
+        assert np.array_equal(same.view(np.uint32), got.view(np.uint32)), (la, lb)
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 1501, 777), (4099, 3841, 89), (1000, 700, 600), (2100, 2300, 100)])
 @pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-36, 1e36), (1e30, 1e-30), (3e-39, 1.0), (1e-20, 1e-19)])
 def test_scales_keep_fp32_accuracy(hip, m, n, k, scale_a, scale_b):
     """Operands of any fp32 scale, subnormals included: the accuracy of the
@@ -93,9 +113,11 @@ def test_scales_keep_fp32_accuracy(hip, m, n, k, scale_a, scale_b):
     a = (rng.standard_normal((m, k)) * scale_a).astype(np.float32)
     b = (rng.standard_normal((k, n)) * scale_b).astype(np.float32)
     print(f"triple scale {scale_a} {scale_b}", flush=True)
-    got = _three_terms(_view(a, "n"), _view(b, "n"))[::8].astype(np.float64)
+    ragged = m % 4 != 0 or n % 4 != 0  # the others are left to the fp32 kernels
+    got = (_three_terms(_view(a, "n"), _view(b, "n")) if ragged else ops.matmul(_view(a, "n"), _view(b, "n")).numpy())
+    got = got[::8].astype(np.float64)
     exact = a[::8].astype(np.float64) @ b.astype(np.float64)
-    terms = min(scale_a, scale_b) > 1e-22  # no input below 2^-110
+    terms = ragged and min(scale_a, scale_b) > 1e-22  # no input below 2^-110
     assert np.linalg.norm(got - exact) <= (_bound(k if terms else 8 * k) * np.linalg.norm(exact)
                                            + 2.0 ** -149 * k * np.sqrt(exact.size))
 
@@ -116,11 +138,11 @@ def test_lower_terms_below_the_smallest_normal_number(hip):
         assert _off(got, exact) <= _bound(k)
 
 
-def test_infinities_nans_and_the_largest_values(hip):
+@pytest.mark.parametrize("m,n,k,terms", [(1100, 1300, 801, True), (600, 640, 800, False)])
+def test_infinities_nans_and_the_largest_values(hip, m, n, k, terms):
     """Where a 64-bit product is finite in fp32, the result is it; elsewhere
     infinities and NaNs land where IEEE arithmetic puts them."""
     rng = np.random.default_rng(SEED)
-    m, n, k = 1100, 1300, 801
     a = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
     b = rng.uniform(0.5, 1.5, (k, n)).astype(np.float32)
     a[3, 5] = np.inf
@@ -131,7 +153,7 @@ def test_infinities_nans_and_the_largest_values(hip):
     b[7, 300] = 0.5
     b[20, 64] = np.inf
     a[200, 20] = 0.0                      # 0 * inf
-    got = _three_terms(_view(a, "n"), _view(b, "n"))
+    got = _three_terms(_view(a, "n"), _view(b, "n")) if terms else ops.matmul(_view(a, "n"), _view(b, "n")).numpy()
     with np.errstate(invalid="ignore", over="ignore"):
         exact = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
     np.testing.assert_array_equal(np.isnan(got), np.isnan(exact))
@@ -142,10 +164,11 @@ def test_infinities_nans_and_the_largest_values(hip):
 
 
 # forward on the 128x128, 64x64 and 256x128 tiles, weight gradient on 64x64,
-# 256x128 and 128x128
-@pytest.mark.parametrize("n,c,hw,cout,window,stride", [(64, 33, (32, 32), 257, 3, 1), (33, 33, (30, 31), 130, 5, 2),
-                                                       (64, 40, (14, 14), 258, 3, 1)])
-def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stride):
+# 256x128 and 128x128; one of both left to the fp32 kernels
+@pytest.mark.parametrize("n,c,hw,cout,window,stride,forward,backward", [
+    (64, 33, (32, 32), 257, 3, 1, 2, 2), (33, 33, (30, 31), 130, 5, 2, 2, 2), (64, 40, (14, 14), 258, 3, 1, 2, 2),
+    (37, 40, (19, 23), 70, 3, 1, 2, 0), (9, 65, (30, 31), 130, 5, 2, 0, 2)])
+def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stride, forward, backward):
     rng = np.random.default_rng(SEED + c)
     x = rng.uniform(-1, 1, (n, c) + hw).astype(np.float32)
     w = rng.uniform(-0.1, 0.1, (cout, c, window, window)).astype(np.float32)
@@ -157,14 +180,14 @@ def test_convolutions_are_the_lowered_products(hip, n, c, hw, cout, window, stri
     with DecisionRecorder() as rec:
         got = ops.conv2d(dx, dw, stride, pad)
         want = ops.matmul(dw.reshape(1, 1, cout, ck).broadcast_to((1, n, cout, ck)), cols.reshape(1, n, ck, L))
-    assert _operand_kinds(rec) == ["three_bf16_terms"] * 2
+    assert _operand_kinds(rec) == ["three_bf16_terms"] * forward
     assert np.array_equal(got.numpy().reshape(-1), want.numpy().reshape(-1))
     g = rng.standard_normal(got.shape).astype(np.float32)
     dg = DeviceArray.from_numpy(g)
     with DecisionRecorder() as rec:
         per = ops.conv2d_weight_grad(dx, dg, window, stride, pad)
         want = ops.matmul(dg.reshape(1, n, cout, L), cols.reshape(1, n, ck, L).transpose(-2, -1)).numpy()
-    assert _operand_kinds(rec) == ["three_bf16_terms"] * 2
+    assert _operand_kinds(rec) == ["three_bf16_terms"] * backward
     assert np.array_equal(per.numpy().reshape(-1), want.reshape(-1))
     total = ops.conv2d_weight_grad_sum(dx, dg, window, stride, pad).numpy()
     exact = np.einsum("nol,nkl->ok", g.reshape(n, cout, L).astype(np.float64), cols.numpy().astype(np.float64),
